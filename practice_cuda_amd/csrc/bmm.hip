@@ -545,18 +545,21 @@ static int bmm_scaled(const void* a, int a_fmt, const void* b, int b_fmt, int64_
     const int64_t b_max = b_k ? (tn * TN) * ldb + kpad : (kpad - 1) * ldb + tn * TN;
     const bool block_ok = scale_mode != PCAMD_SCALE_BLOCK ||
                           (args.qbm_shift >= 0 && args.qbn_shift >= 0);
-    const bool fast = k > 0 && (!ragged || wide) && args.vec_a && args.vec_b && lda % 16 == 0 && ldb % 16 == 0 &&
-                      a_max < (int64_t{1} << 32) - 64 && b_max < (int64_t{1} << 32) - 64 &&
-                      m < INT32_MAX && n < INT32_MAX && k < INT32_MAX && tm * tn * batch < INT32_MAX &&
-                      block_ok && !env_generic;
-    if (fast) {
+    // sizes and offsets fit the 32-bit fields of FastArgs
+    const int64_t a_ext = a_k ? (m - 1) * sam + k : (k - 1) * sak + m;
+    const int64_t b_ext = b_k ? (n - 1) * sbn + k : (k - 1) * sbk + n;
+    const bool small = k > 0 && lda >= 0 && ldb >= 0 && a_ext <= UINT32_MAX && b_ext <= UINT32_MAX && m < INT32_MAX &&
+                       n < INT32_MAX && k < INT32_MAX - 256 && tm * tn * batch < INT32_MAX && block_ok && !env_generic;
+    const bool fast = small && (!ragged || wide) && args.vec_a && args.vec_b && lda % 16 == 0 && ldb % 16 == 0 &&
+                      a_max < (int64_t{1} << 32) - 64 && b_max < (int64_t{1} << 32) - 64;
+    if (small) {
       FastArgs f{};
       f.a = args.a; f.b = args.b; f.c = c; f.bias = bias; f.sa = sa; f.sb = sb;
       f.m = static_cast<int32_t>(m); f.n = static_cast<int32_t>(n); f.k = static_cast<int32_t>(k);
       f.sab = sab; f.sbb = sbb;
       f.lda = static_cast<uint32_t>(lda); f.ldb = static_cast<uint32_t>(ldb);
-      f.a_extent = static_cast<uint32_t>(a_k ? (m - 1) * sam + k : (k - 1) * sak + m);
-      f.b_extent = static_cast<uint32_t>(b_k ? (n - 1) * sbn + k : (k - 1) * sbk + n);
+      f.a_extent = static_cast<uint32_t>(a_ext);
+      f.b_extent = static_cast<uint32_t>(b_ext);
       f.scb = scb; f.scm = scm; f.scn = scn;
       f.sbiasb = sbiasb; f.sbiasm = sbiasm; f.sbiasn = sbiasn;
       f.ssab = ssab; f.ssa1 = ssa1; f.ssa2 = ssa2; f.ssbb = ssbb; f.ssb1 = ssb1; f.ssb2 = ssb2;
@@ -569,10 +572,15 @@ static int bmm_scaled(const void* a, int a_fmt, const void* b, int b_fmt, int64_
       const bool sb_col = scale_mode == PCAMD_SCALE_BLOCK && args.qbn < 16;
       const bool qb1 = scale_mode == PCAMD_SCALE_BLOCK && args.qbk == 128;
       // the streaming (config-4) and 128 x 256 kernels take one format for both operands
-      if (same_fmt && !env_no_stream && bmm_stream_ok(f, a_k, b_k, fmode, batch, args.qbm, args.qbn, ssa1, ssb2))
+      if (fast && same_fmt && !env_no_stream &&
+          bmm_stream_ok(f, a_k, b_k, fmode, batch, args.qbm, args.qbn, ssa1, ssb2))
         return bmm_stream_launch(f, a_fmt, batch, st);
-      if (wide) return bmm_wide_launch(f, a_fmt, b_fmt, a_k, b_k, fmode, st);
-      if (same_fmt) return bmm_fast_launch(f, a_fmt, a_k, b_k, fmode, sb_col, qb1, st);
+      // products of several K steps on a short grid, and unaligned operands
+      if (bmm_split_ok(f, a_fmt, b_fmt, a_k, b_k, fmode, batch) &&
+          (!fast || (wide && bmm_split_pays(f, batch, st))))
+        return bmm_split_launch(f, a_k, b_k, fmode, batch, st);
+      if (fast && wide) return bmm_wide_launch(f, a_fmt, b_fmt, a_k, b_k, fmode, st);
+      if (fast && same_fmt) return bmm_fast_launch(f, a_fmt, a_k, b_k, fmode, sb_col, qb1, st);
     }
   }
   return bmm::launch_formats(args, a_fmt, b_fmt, a_k, b_k, mode, st);
