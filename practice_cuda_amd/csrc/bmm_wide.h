@@ -612,14 +612,14 @@ __global__ __launch_bounds__(NT, 1) void bmm_wide_kernel(FastArgs a) {
       // barrier is needed)
       const float sam_v[4] = {row_scale(0), row_scale(1), row_scale(2), row_scale(3)};
       uint16_t* cb = reinterpret_cast<uint16_t*>(a.c) + bidx * a.scb;
-      auto stage = [&](auto out_c, auto&& value) {
+      auto stage = [&](auto out_c, auto&& value, auto bias) {
         constexpr int OUT = decltype(out_c)::value;
         if constexpr (JN == 8)
           store_subtile_staged<OUT>(smem + (ksteps & 1) * STAGE + wave * 8192, cb, a.scm, a.m, a.n, m0 + wm * 64,
-                                    n0 + wcol, lane, value, a.c_dtype == kF16);
+                                    n0 + wcol, lane, value, a.c_dtype == kF16, bias);
         else
           store_half_staged<OUT>(smem + (ksteps & 1) * STAGE + wave * 4096, cb, a.scm, a.m, a.n, m0 + wm * 64,
-                                 n0 + wcol, lane, value, a.c_dtype == kF16);
+                                 n0 + wcol, lane, value, a.c_dtype == kF16, bias);
       };
       if constexpr (CT) {
         // every wave's 14 KiB of staging spans both LDS stages: wait until all
@@ -642,36 +642,56 @@ __global__ __launch_bounds__(NT, 1) void bmm_wide_kernel(FastArgs a) {
             col_scales(j, sbv);
 #pragma unroll
             for (int r = 0; r < 4; ++r) v[r] = out_value(i, j, r, sam_v[i], sbv);
-          });
+          }, NoBias{});
           return;
         }
         // fp16 output, a 16-bit bias and / or GELU, in the reference's order:
         // scaled product, + bias, activation, one rounding
         // (kernels/bmm/per_block.py:113-137). The output type is picked per
-        // element pair at run time (OUT16_RUNTIME), so this path is
-        // instantiated once.
+        // element pair at run time (OUT16_RUNTIME); with and without a bias
+        // are two instantiations, as the bias takes registers.
         const bool bias_bf16 = a.bias_dtype == kBF16, gelu = a.act == PCAMD_ACT_GELU;
-        const uint16_t* bias_b = bias16 ? static_cast<const uint16_t*>(a.bias) + bidx * a.sbiasb : nullptr;
         auto value = [&](int i, int j, float (&v)[4]) {
           float sbv[4];
           col_scales(j, sbv);
 #pragma unroll
           for (int r = 0; r < 4; ++r) v[r] = out_value(i, j, r, sam_v[i], sbv);
-          const int mm = row_base + 16 * i, nn = col_base + 16 * j;
-          if (bias_b && mm < a.m && nn < a.n) {
-            const uint2 h = *reinterpret_cast<const uint2*>(bias_b + int64_t(mm) * a.sbiasm + nn);
-            const uint32_t e[4] = {h.x & 0xFFFFu, h.x >> 16, h.y & 0xFFFFu, h.y >> 16};
-#pragma unroll
-            for (int r = 0; r < 4; ++r)
-              v[r] += bias_bf16 ? __uint_as_float(e[r] << 16)
-                                : static_cast<float>(__builtin_bit_cast(_Float16, static_cast<uint16_t>(e[r])));
-          }
+        };
+        auto activate = [&](float (&v)[4]) {
           if (gelu) {
 #pragma unroll
             for (int r = 0; r < 4; ++r) v[r] = 0.5f * v[r] * (1.0f + erff(v[r] * 0.7071067811865475f));
           }
         };
-        stage(IC<OUT16_RUNTIME>{}, value);
+        auto add_bias = [&](float (&v)[4], const uint2& h) {
+          v[0] += bias_bf16 ? bf16_lo(h.x) : f16_lo(h.x);
+          v[1] += bias_bf16 ? bf16_hi(h.x) : f16_hi(h.x);
+          v[2] += bias_bf16 ? bf16_lo(h.y) : f16_lo(h.y);
+          v[3] += bias_bf16 ? bf16_hi(h.y) : f16_hi(h.y);
+        };
+        const RowBias rb{static_cast<const uint16_t*>(a.bias) + bidx * a.sbiasb, a.sbiasm};
+        if (a.bias != nullptr) {
+          if constexpr (MODE == 0 && SBK == 2) {
+            // the per-column scales leave no registers for the row loads: 8 bytes per lane
+            stage(IC<OUT16_RUNTIME>{}, [&](int i, int j, float (&v)[4]) {
+              value(i, j, v);
+              const int mm = row_base + 16 * i, nn = col_base + 16 * j;
+              if (mm < a.m && nn < a.n) add_bias(v, *reinterpret_cast<const uint2*>(rb.p + mm * rb.row_stride + nn));
+              activate(v);
+            }, NoBias{});
+          } else {
+            stage(IC<OUT16_RUNTIME>{}, [&](int i, int j, float (&v)[4], const uint2& h) {
+              value(i, j, v);
+              add_bias(v, h);
+              activate(v);
+            }, rb);
+          }
+        } else {
+          stage(IC<OUT16_RUNTIME>{}, [&](int i, int j, float (&v)[4]) {
+            value(i, j, v);
+            activate(v);
+          }, NoBias{});
+        }
         return;
       }
     }
