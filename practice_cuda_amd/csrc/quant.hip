@@ -32,6 +32,8 @@
 //   quant_cols_kernel   whole columns of up to 256 rows (channel_axis = -1,
 //                       two passes over the strip), and column groups on grids
 //                       too large for the column-group kernel's 3-D grid.
+//   (the group, row, tile, per-column and per-tensor kernels also take
+//                       contiguous rows of any length and alignment: UA)
 //   quant_*_generic     any strides / block shape; one workgroup per block or
 //                       channel, two passes (second read served by L2).
 //   per-tensor          amax kernel (workgroup max + one atomic max on the
@@ -72,7 +74,7 @@ struct RowArgs {
   float* scale;
   int64_t total;    // chunks of the whole tensor (flat group kernel)
   uint32_t units;   // rows * segs
-  int32_t chunks;   // 8-element chunks per row
+  int32_t chunks;   // 8-element chunks per row (the last one may be partial in UA kernels)
   float fp8_max, eps;
   uint32_t m;       // rows per batch
   uint32_t segs;    // segments per row (group kernel)
@@ -80,6 +82,7 @@ struct RowArgs {
   int64_t sxb, sxm; // input strides (elements)
   int64_t syb, sym; // output strides (bytes == elements)
   int64_t ssb, ssm, ssn;  // scale strides (elements)
+  int64_t n;              // elements per row (UA kernels)
 };
 static_assert(offsetof(RowArgs, eps) + sizeof(float) <= 64, "flat group kernel fields in one 64-byte line");
 
@@ -95,6 +98,49 @@ PCAMD_DEV void store8(uint8_t* p, uint2 v) {
   }
 }
 
+// Rows of any length at any element address (UA): a chunk is loaded and stored
+// whole without alignment (global loads and stores take any address), a row's
+// last one, of nv < 8 elements, element by element. Their stores allocate in
+// cache: rows end inside cache lines, which neighbouring rows complete.
+template <int EB> struct __attribute__((packed, aligned(EB))) RawChunk { u32x4_t r[EB == 4 ? 2 : 1]; };
+struct __attribute__((packed)) RawOut { u32x2 v; };
+
+template <int DT, bool UA>
+PCAMD_DEV void load_chunk_n(Chunk<DT>& c, const char* p, int64_t nv) {
+  if constexpr (!UA) {
+    load_chunk<DT>(c, p);
+  } else if (nv >= 8) {
+    constexpr int EB = elem_bytes<DT>();
+    const RawChunk<EB> t = *reinterpret_cast<const RawChunk<EB>*>(p);
+#pragma unroll
+    for (int h = 0; h < (DT == kF32 ? 2 : 1); ++h) c.r[h] = make_uint4(t.r[h].x, t.r[h].y, t.r[h].z, t.r[h].w);
+  } else {
+    uint32_t w[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+#pragma unroll
+    for (int e = 0; e < 7; ++e) {
+      if (e < nv) {
+        if constexpr (DT == kF32) w[e] = reinterpret_cast<const uint32_t*>(p)[e];
+        else w[e >> 1] |= static_cast<uint32_t>(reinterpret_cast<const uint16_t*>(p)[e]) << (16 * (e & 1));
+      }
+    }
+    c.r[0] = make_uint4(w[0], w[1], w[2], w[3]);
+    if constexpr (DT == kF32) c.r[1] = make_uint4(w[4], w[5], w[6], w[7]);
+  }
+}
+
+template <int DT, bool NTS, bool UA>
+PCAMD_DEV void store8_n(uint8_t* p, uint2 v, int64_t nv) {
+  if constexpr (!UA) {
+    store8<DT, NTS>(p, v);
+  } else if (nv >= 8) {
+    reinterpret_cast<RawOut*>(p)->v = u32x2{v.x, v.y};
+  } else {
+#pragma unroll
+    for (int e = 0; e < 7; ++e)
+      if (e < nv) p[e] = static_cast<uint8_t>((e < 4 ? v.x : v.y) >> (8 * (e & 3)));
+  }
+}
+
 // 1 x (8 * LPG) groups along a row. A unit is CPL * 64 consecutive chunks of
 // one row; each wave quantizes one unit (kGroupThreads / 64 units per
 // workgroup). FLAT: input, output and scales are contiguous and the row
@@ -107,7 +153,7 @@ constexpr int kGroupThreads = 256;
 // the per-tensor quantize pass keeps its measured 128-thread workgroups
 constexpr int kTensorFlatThreads = 128;
 
-template <int DT, int FMT, int LPG, int CPL, bool NTS, bool FLAT, bool CLAMP>
+template <int DT, int FMT, int LPG, int CPL, bool NTS, bool FLAT, bool CLAMP, bool UA = false>
 __global__ __launch_bounds__(kGroupThreads) void quant_groups_kernel(RowArgs a) {
   constexpr int EB = elem_bytes<DT>();
   const int lane = threadIdx.x & 63;
@@ -142,7 +188,7 @@ __global__ __launch_bounds__(kGroupThreads) void quant_groups_kernel(RowArgs a) 
 #pragma unroll
   for (int c = 0; c < CPL; ++c) {
     const int ch = chunk0 + c * 64;
-    if (ch < a.chunks) load_chunk<DT>(cur[c], xrow + int64_t(ch) * 8 * EB);
+    if (ch < a.chunks) load_chunk_n<DT, UA>(cur[c], xrow + int64_t(ch) * 8 * EB, a.n - int64_t(ch) * 8);
     else zero_chunk<DT>(cur[c]);
   }
   uint8_t* yrow = a.y + int64_t(b) * a.syb + int64_t(mi) * a.sym;
@@ -154,14 +200,15 @@ __global__ __launch_bounds__(kGroupThreads) void quant_groups_kernel(RowArgs a) 
     const Scales s = block_scales(amax, a.fp8_max, a.eps);
     if (ch < a.chunks) {
       if ((lane & (LPG - 1)) == 0) srow[int64_t(ch / LPG) * a.ssn] = s.ds;
-      store8<DT, NTS>(yrow + int64_t(ch) * 8, quant_chunk<DT, FMT, CLAMP>(cur[c], s.qs, a.fp8_max));
+      store8_n<DT, NTS, UA>(yrow + int64_t(ch) * 8, quant_chunk<DT, FMT, CLAMP>(cur[c], s.qs, a.fp8_max),
+                            a.n - int64_t(ch) * 8);
     }
   }
 }
 
 // Per-channel along the row, one wave per row: the row (up to 64 * MAXC
 // chunks) is held in registers and read from HBM once.
-template <int DT, int FMT, int MAXC, bool NTS>
+template <int DT, int FMT, int MAXC, bool NTS, bool UA = false>
 __global__ __launch_bounds__(kThreads) void quant_waverow_kernel(RowArgs a) {
   constexpr int EB = elem_bytes<DT>();
   const int lane = threadIdx.x & 63;
@@ -173,7 +220,7 @@ __global__ __launch_bounds__(kThreads) void quant_waverow_kernel(RowArgs a) {
 #pragma unroll
   for (int c = 0; c < MAXC; ++c) {
     const int ch = lane + c * 64;
-    if (c < a.cpl && ch < a.chunks) load_chunk<DT>(raw[c], xrow + int64_t(ch) * 8 * EB);
+    if (c < a.cpl && ch < a.chunks) load_chunk_n<DT, UA>(raw[c], xrow + int64_t(ch) * 8 * EB, a.n - int64_t(ch) * 8);
     else zero_chunk<DT>(raw[c]);
   }
   float amax = 0.0f;
@@ -187,7 +234,8 @@ __global__ __launch_bounds__(kThreads) void quant_waverow_kernel(RowArgs a) {
   for (int c = 0; c < MAXC; ++c) {
     const int ch = lane + c * 64;
     if (c < a.cpl && ch < a.chunks)
-      store8<DT, NTS>(yrow + int64_t(ch) * 8, quant_chunk<DT, FMT>(raw[c], s.qs, a.fp8_max));
+      store8_n<DT, NTS, UA>(yrow + int64_t(ch) * 8, quant_chunk<DT, FMT>(raw[c], s.qs, a.fp8_max),
+                            a.n - int64_t(ch) * 8);
   }
 }
 
@@ -197,7 +245,7 @@ __global__ __launch_bounds__(kThreads) void quant_waverow_kernel(RowArgs a) {
 // GRID2: grid (rows, batch), so the row and batch come from the workgroup
 // index with no division ahead of the loads; otherwise a 1-D grid of
 // batch * rows.
-template <int DT, int FMT, int CPT, bool NTS, bool GRID2, bool CLAMP>
+template <int DT, int FMT, int CPT, bool NTS, bool GRID2, bool CLAMP, bool UA = false>
 __global__ __launch_bounds__(1024) void quant_rowblock_kernel(RowArgs a) {
   constexpr int EB = elem_bytes<DT>();
   __shared__ float red[1024 / 64];
@@ -215,7 +263,7 @@ __global__ __launch_bounds__(1024) void quant_rowblock_kernel(RowArgs a) {
 #pragma unroll
   for (int c = 0; c < CPT; ++c) {
     const int ch = t + c * nt;
-    if (ch < a.chunks) load_chunk<DT>(cur[c], xrow + int64_t(ch) * 8 * EB);
+    if (ch < a.chunks) load_chunk_n<DT, UA>(cur[c], xrow + int64_t(ch) * 8 * EB, a.n - int64_t(ch) * 8);
     else zero_chunk<DT>(cur[c]);
   }
   float amax = 0.0f;
@@ -233,7 +281,8 @@ __global__ __launch_bounds__(1024) void quant_rowblock_kernel(RowArgs a) {
   for (int c = 0; c < CPT; ++c) {
     const int ch = t + c * nt;
     if (ch < a.chunks)
-      store8<DT, NTS>(yrow + int64_t(ch) * 8, quant_chunk<DT, FMT, CLAMP>(cur[c], s.qs, a.fp8_max));
+      store8_n<DT, NTS, UA>(yrow + int64_t(ch) * 8, quant_chunk<DT, FMT, CLAMP>(cur[c], s.qs, a.fp8_max),
+                            a.n - int64_t(ch) * 8);
   }
 }
 
@@ -252,6 +301,7 @@ struct TileArgs {
   int32_t block_m;
   int32_t cpt;       // chunks per thread = block_m * lpr / 256
   int32_t lpr, lpr_shift;  // lanes per block row (block_n / 8) and its log2
+  int32_t any;       // rows of any length and alignment
   int32_t wide;      // H > 0: 128 x 128 blocks, 4 H per workgroup (quant_tile_wide_kernel)
   float fp8_max, eps;
 };
@@ -260,7 +310,7 @@ struct TileArgs {
 // m, batch) and the block comes from the workgroup index; otherwise the grid
 // is 1-D (capped) and workgroups stride over the flattened block index. FULL:
 // m and n are multiples of the block, so no row / column bounds checks.
-template <int DT, int FMT, int CPT, bool NTS, bool GRID3, bool FULL, bool CLAMP>
+template <int DT, int FMT, int CPT, bool NTS, bool GRID3, bool FULL, bool CLAMP, bool UA = false>
 __global__ __launch_bounds__(kThreads) void quant_tile_kernel(TileArgs a) {
   constexpr int EB = elem_bytes<DT>();
   __shared__ float red[2][kThreads / 64];
@@ -276,7 +326,7 @@ __global__ __launch_bounds__(kThreads) void quant_tile_kernel(TileArgs a) {
 #pragma unroll
     for (int p = 0; p < CPT; ++p) {
       const int64_t r = r0 + p * rpp + rp;
-      if (FULL || (r < a.m && col < a.n)) load_chunk<DT>(cur[p], xb + (r * a.sxm + col) * EB);
+      if (FULL || (r < a.m && col < a.n)) load_chunk_n<DT, UA>(cur[p], xb + (r * a.sxm + col) * EB, a.n - col);
       else zero_chunk<DT>(cur[p]);
     }
     float amax = 0.0f;
@@ -293,7 +343,7 @@ __global__ __launch_bounds__(kThreads) void quant_tile_kernel(TileArgs a) {
     for (int p = 0; p < CPT; ++p) {
       const int64_t r = r0 + p * rpp + rp;
       if (FULL || (r < a.m && col < a.n))
-        store8<DT, NTS>(yb + r * a.sym + col, quant_chunk<DT, FMT, CLAMP>(cur[p], s.qs, a.fp8_max));
+        store8_n<DT, NTS, UA>(yb + r * a.sym + col, quant_chunk<DT, FMT, CLAMP>(cur[p], s.qs, a.fp8_max), a.n - col);
     }
   };
   if constexpr (GRID3) {
@@ -625,11 +675,11 @@ __global__ __launch_bounds__(kThreads) void tensor_quant_kernel(TensorArgs a) {
 constexpr int kAmaxThreads = 512;
 constexpr int kAmaxGrid = 256;
 
-template <int DT>
+template <int DT, bool UA = false>
 __global__ __launch_bounds__(kAmaxThreads) void tensor_amax_flat_kernel(TensorArgs a) {
   constexpr int EB = elem_bytes<DT>(), CPT = 8, W = kAmaxThreads / 64;
   __shared__ float red[W];
-  const int64_t chunks = a.total / 8;
+  const int64_t chunks = (a.total + 7) / 8;
   constexpr int64_t kUnit = int64_t(kAmaxThreads) * CPT;
   float amax = 0.0f;
   for (int64_t base = int64_t(blockIdx.x) * kUnit; base < chunks; base += int64_t(gridDim.x) * kUnit) {
@@ -637,7 +687,7 @@ __global__ __launch_bounds__(kAmaxThreads) void tensor_amax_flat_kernel(TensorAr
 #pragma unroll
     for (int p = 0; p < CPT; ++p) {
       const int64_t ch = base + p * kAmaxThreads + threadIdx.x;
-      if (ch < chunks) load_chunk<DT>(c[p], a.x + ch * 8 * EB);
+      if (ch < chunks) load_chunk_n<DT, UA>(c[p], a.x + ch * 8 * EB, a.total - ch * 8);
       else zero_chunk<DT>(c[p]);
     }
 #pragma unroll
@@ -653,10 +703,10 @@ __global__ __launch_bounds__(kAmaxThreads) void tensor_amax_flat_kernel(TensorAr
   }
 }
 
-template <int DT, int FMT, bool NTS>
+template <int DT, int FMT, bool NTS, bool UA = false>
 __global__ __launch_bounds__(kTensorFlatThreads) void tensor_quant_flat_kernel(TensorArgs a) {
   constexpr int EB = elem_bytes<DT>(), CPL = 2;
-  const int64_t chunks = a.total / 8;
+  const int64_t chunks = (a.total + 7) / 8;
   const int lane = threadIdx.x & 63;
   const int64_t u = int64_t(blockIdx.x) * (kTensorFlatThreads / 64) + (threadIdx.x >> 6);
   const int64_t ch0 = u * (CPL * 64) + lane;
@@ -664,7 +714,7 @@ __global__ __launch_bounds__(kTensorFlatThreads) void tensor_quant_flat_kernel(T
 #pragma unroll
   for (int c = 0; c < CPL; ++c) {
     const int64_t ch = ch0 + c * 64;
-    if (ch < chunks) load_chunk<DT>(cur[c], a.x + ch * 8 * EB);
+    if (ch < chunks) load_chunk_n<DT, UA>(cur[c], a.x + ch * 8 * EB, a.total - ch * 8);
     else zero_chunk<DT>(cur[c]);
   }
   const Scales s = tensor_scales(__uint_as_float(*reinterpret_cast<const uint32_t*>(a.scale)), a.fp8_max, a.eps,
@@ -672,7 +722,8 @@ __global__ __launch_bounds__(kTensorFlatThreads) void tensor_quant_flat_kernel(T
 #pragma unroll
   for (int c = 0; c < CPL; ++c) {
     const int64_t ch = ch0 + c * 64;
-    if (ch < chunks) store8<DT, NTS>(a.y + ch * 8, quant_chunk<DT, FMT>(cur[c], s.qs, a.fp8_max));
+    if (ch < chunks)
+      store8_n<DT, NTS, UA>(a.y + ch * 8, quant_chunk<DT, FMT>(cur[c], s.qs, a.fp8_max), a.total - ch * 8);
   }
 }
 
@@ -819,7 +870,7 @@ __global__ __launch_bounds__(kThreads) void colchan_zero_kernel(ColArgs a) {
 // ordinary (temporal) loads, unlike the other kernels: the apply kernel
 // reads it again right after, and what the caches keep of it saves HBM
 // reads ([18432, 7168] bf16: 117 -> 106 us for the pair).
-template <int DT>
+template <int DT, bool UA = false>
 __global__ __launch_bounds__(kThreads) void colchan_amax_kernel(ColArgs a) {
   constexpr int EB = elem_bytes<DT>();
   constexpr int CPT = 8, WAVES = kThreads / 64;
@@ -834,8 +885,12 @@ __global__ __launch_bounds__(kThreads) void colchan_amax_kernel(ColArgs a) {
 #pragma unroll
   for (int p = 0; p < CPT; ++p) {
     const int64_t r = r0 + p * 16 + rs;
-    if (r < a.m && col < a.n) load_chunk_temporal<DT>(raw[p], xb + (r * a.sxm + col) * EB);
-    else zero_chunk<DT>(raw[p]);
+    if (r < a.m && col < a.n) {
+      if constexpr (UA) load_chunk_n<DT, true>(raw[p], xb + (r * a.sxm + col) * EB, a.n - col);
+      else load_chunk_temporal<DT>(raw[p], xb + (r * a.sxm + col) * EB);
+    } else {
+      zero_chunk<DT>(raw[p]);
+    }
   }
   float cmax[8] = {0, 0, 0, 0, 0, 0, 0, 0};
 #pragma unroll
@@ -865,7 +920,7 @@ __global__ __launch_bounds__(kThreads) void colchan_amax_kernel(ColArgs a) {
 }
 
 // Same grid: quantize the slab with the finished column maxima.
-template <int DT, int FMT, bool NTS>
+template <int DT, int FMT, bool NTS, bool UA = false>
 __global__ __launch_bounds__(kThreads) void colchan_apply_kernel(ColArgs a) {
   constexpr int EB = elem_bytes<DT>();
   constexpr int CPT = 8;
@@ -880,7 +935,7 @@ __global__ __launch_bounds__(kThreads) void colchan_apply_kernel(ColArgs a) {
 #pragma unroll
   for (int p = 0; p < CPT; ++p) {
     const int64_t r = r0 + p * 16 + rs;
-    if (r < a.m && col_ok) load_chunk<DT>(raw[p], xb + (r * a.sxm + col) * EB);
+    if (r < a.m && col_ok) load_chunk_n<DT, UA>(raw[p], xb + (r * a.sxm + col) * EB, a.n - col);
     else zero_chunk<DT>(raw[p]);
   }
   // one division per column of the strip (lanes t < 128), shared through LDS
@@ -903,8 +958,9 @@ __global__ __launch_bounds__(kThreads) void colchan_apply_kernel(ColArgs a) {
       unpack_chunk<DT>(raw[p], v);
 #pragma unroll
       for (int i = 0; i < 8; ++i) v[i] = clamp_sym(v[i] * qs[i], a.fp8_max);
-      store8<DT, NTS>(yb + r * a.sym + col,
-                      make_uint2(pack4<FMT>(v[0], v[1], v[2], v[3]), pack4<FMT>(v[4], v[5], v[6], v[7])));
+      store8_n<DT, NTS, UA>(yb + r * a.sym + col,
+                            make_uint2(pack4<FMT>(v[0], v[1], v[2], v[3]), pack4<FMT>(v[4], v[5], v[6], v[7])),
+                            a.n - col);
     }
   }
 }
@@ -1209,6 +1265,25 @@ struct LaunchGroups {
   }
   template <bool NTS>
   static int by_lpg(const RowArgs& a, int lpg, int cpl, hipStream_t st) {
+    // rows of any length and alignment: the two-chunk unit, cached stores
+    if (a.n > 0) {
+      constexpr int kWaves = kGroupThreads / 64;
+      const int grid = static_cast<int>((int64_t(a.units) + kWaves - 1) / kWaves);
+      auto ua = [&](auto l) {
+        quant_groups_kernel<DT, FMT, decltype(l)::value, 2, false, false, true, true>
+            <<<grid, kGroupThreads, 0, st>>>(a);
+        return check_launch("quant_groups_kernel");
+      };
+      switch (lpg) {
+        case 1: return ua(std::integral_constant<int, 1>{});
+        case 2: return ua(std::integral_constant<int, 2>{});
+        case 4: return ua(std::integral_constant<int, 4>{});
+        case 8: return ua(std::integral_constant<int, 8>{});
+        case 16: return ua(std::integral_constant<int, 16>{});
+        case 32: return ua(std::integral_constant<int, 32>{});
+        default: return ua(std::integral_constant<int, 64>{});
+      }
+    }
     switch (lpg) {
       case 1: return by_cpl<1, NTS>(a, cpl, st);
       case 2: return by_cpl<2, NTS>(a, cpl, st);
@@ -1260,7 +1335,18 @@ struct LaunchRowBlock {
     if (a.chunks <= 512) return go<2, NTS>(a, ((a.chunks + 1) / 2 + 63) / 64 * 64, st);
     return go<4, NTS>(a, ((a.chunks + 3) / 4 + 63) / 64 * 64, st);  // <= 512 threads: chunks <= 2048
   }
-  static int run(const RowArgs& a, hipStream_t st) { return nt_stores() ? pick<true>(a, st) : pick<false>(a, st); }
+  static int run(const RowArgs& a, hipStream_t st) {
+    if (a.n > 0) {  // rows of any length and alignment
+      if (a.chunks < 256) {
+        quant_waverow_kernel<DT, FMT, 4, false, true><<<static_cast<int>((int64_t(a.units) + 3) / 4), kThreads, 0, st>>>(a);
+        return check_launch("quant_waverow_kernel");
+      }
+      const int threads = ((a.chunks + 3) / 4 + 63) / 64 * 64;
+      quant_rowblock_kernel<DT, FMT, 4, false, false, true, true><<<a.units, threads, 0, st>>>(a);
+      return check_launch("quant_rowblock_kernel");
+    }
+    return nt_stores() ? pick<true>(a, st) : pick<false>(a, st);
+  }
 };
 
 template <int DT, int FMT>
@@ -1311,7 +1397,22 @@ struct LaunchTile {
       default: return set_error(PCAMD_ERR_UNSUPPORTED, "tile kernel: unsupported chunks per thread %d", a.cpt);
     }
   }
+  template <int CPT>
+  static int any(const TileArgs& a, hipStream_t st) {
+    quant_tile_kernel<DT, FMT, CPT, false, false, false, true, true><<<grid_for(a.blocks), kThreads, 0, st>>>(a);
+    return check_launch("quant_tile_kernel");
+  }
   static int run(const TileArgs& a, hipStream_t st) {
+    if (a.any) {  // rows of any length and alignment
+      switch (a.cpt) {
+        case 1: return any<1>(a, st);
+        case 2: return any<2>(a, st);
+        case 4: return any<4>(a, st);
+        case 8: return any<8>(a, st);
+        case 16: return any<16>(a, st);
+        default: return set_error(PCAMD_ERR_UNSUPPORTED, "tile kernel: unsupported chunks per thread %d", a.cpt);
+      }
+    }
     if (a.wide == 2) return run_wide<2>(a, st);
     if (a.wide == 1) return run_wide<1>(a, st);
     return nt_stores() ? by_cpt<true>(a, st) : by_cpt<false>(a, st);
@@ -1369,19 +1470,20 @@ struct LaunchDual {
 
 template <int DT, int FMT>
 struct LaunchColChan {
-  template <bool NTS>
+  template <bool NTS, bool UA>
   static int go(const ColArgs& a, int64_t batch, hipStream_t st) {
     const int lin = static_cast<int>((batch * a.n + kThreads - 1) / kThreads);
     const dim3 grid(static_cast<uint32_t>(a.strips), static_cast<uint32_t>((a.m + 127) / 128),
                     static_cast<uint32_t>(batch));
     colchan_zero_kernel<<<lin, kThreads, 0, st>>>(a);
-    colchan_amax_kernel<DT><<<grid, kThreads, 0, st>>>(a);
-    colchan_apply_kernel<DT, FMT, NTS><<<grid, kThreads, 0, st>>>(a);
+    colchan_amax_kernel<DT, UA><<<grid, kThreads, 0, st>>>(a);
+    colchan_apply_kernel<DT, FMT, NTS, UA><<<grid, kThreads, 0, st>>>(a);
     colchan_finalize_kernel<<<lin, kThreads, 0, st>>>(a);
     return check_launch("per-column kernels");
   }
-  static int run(const ColArgs& a, int64_t batch, hipStream_t st) {
-    return nt_stores() ? go<true>(a, batch, st) : go<false>(a, batch, st);
+  static int run(const ColArgs& a, int64_t batch, bool any, hipStream_t st) {
+    if (any) return go<false, true>(a, batch, st);
+    return nt_stores() ? go<true, false>(a, batch, st) : go<false, false>(a, batch, st);
   }
 };
 
@@ -1408,14 +1510,18 @@ struct LaunchGeneric {
 
 template <int DT, int FMT>
 struct LaunchTensor {
-  static int run(const TensorArgs& a, bool flat, hipStream_t st) {
+  // flat: one contiguous run of elements; any: not of whole aligned chunks
+  static int run(const TensorArgs& a, bool flat, bool any, hipStream_t st) {
     fill_zero_u32_kernel<<<1, 1, 0, st>>>(reinterpret_cast<uint32_t*>(a.scale));
     if (a.total > 0 && flat) {
-      const int64_t chunks = a.total / 8;
-      tensor_amax_flat_kernel<DT><<<grid_for(chunks, kAmaxThreads * 8, kAmaxGrid), kAmaxThreads, 0, st>>>(a);
+      const int64_t chunks = (a.total + 7) / 8;
+      const int agrid = grid_for(chunks, kAmaxThreads * 8, kAmaxGrid);
+      if (any) tensor_amax_flat_kernel<DT, true><<<agrid, kAmaxThreads, 0, st>>>(a);
+      else tensor_amax_flat_kernel<DT><<<agrid, kAmaxThreads, 0, st>>>(a);
       const int64_t waves = (chunks + 127) / 128;
       const int grid = static_cast<int>((waves + kTensorFlatThreads / 64 - 1) / (kTensorFlatThreads / 64));
-      if (nt_stores()) tensor_quant_flat_kernel<DT, FMT, true><<<grid, kTensorFlatThreads, 0, st>>>(a);
+      if (any) tensor_quant_flat_kernel<DT, FMT, false, true><<<grid, kTensorFlatThreads, 0, st>>>(a);
+      else if (nt_stores()) tensor_quant_flat_kernel<DT, FMT, true><<<grid, kTensorFlatThreads, 0, st>>>(a);
       else tensor_quant_flat_kernel<DT, FMT, false><<<grid, kTensorFlatThreads, 0, st>>>(a);
     } else if (a.total > 0) {
       const int grid = grid_for(a.total, kThreads, 4096);
@@ -1438,6 +1544,12 @@ inline bool row_fast_ok(const void* x, int dt, const void* y, int64_t n, int64_t
   return sxn == 1 && syn == 1 && n % 8 == 0 && aligned(x, 16) && aligned(y, 8) && sxb % vec == 0 &&
          sxm % vec == 0 && syb % 8 == 0 && sym % 8 == 0;
 }
+
+// rows contiguous in input and output, of any length, pitch and alignment
+// (the element-wise kernels divide per element and load 2 bytes at a time; MI355X,
+// bf16 [3, 1001, 1031] quantized in 1 x 128 groups, then a product: 75.9 -> 42.2
+// us per pair of calls)
+inline bool row_any_ok(int64_t n, int64_t sxn, int64_t syn) { return sxn == 1 && syn == 1 && n > 0; }
 
 int validate_common(const void* x, int x_dtype, int64_t batch, int64_t m, int64_t n, const void* y,
                     int y_dtype, const void* scale, float fp8_max) {
@@ -1469,15 +1581,16 @@ extern "C" int pcamd_quant_block(const void* x, int x_dtype, int64_t batch, int6
   if (batch == 0 || m == 0 || n == 0) return PCAMD_OK;
   hipStream_t st = static_cast<hipStream_t>(stream);
   const bool fast = row_fast_ok(x, x_dtype, y, n, sxb, sxm, sxn, syb, sym, syn);
+  const bool rows = fast || row_any_ok(n, sxn, syn);
   const int64_t mb = (m + block_m - 1) / block_m, nb = (n + block_n - 1) / block_n;
 
-  if (fast && block_m == 1 && block_n >= 8 && block_n <= 512 && batch * m < UINT32_MAX / 64 &&
+  if (rows && block_m == 1 && block_n >= 8 && block_n <= 512 && batch * m < UINT32_MAX / 64 &&
       m < UINT32_MAX && n / 8 < INT32_MAX / 2) {
     RowArgs a{};
     a.x = static_cast<const char*>(x); a.y = static_cast<uint8_t*>(y); a.scale = scale;
     a.m = static_cast<uint32_t>(m); a.sxb = sxb; a.sxm = sxm; a.syb = syb; a.sym = sym;
     a.ssb = ssb; a.ssm = ssm; a.ssn = ssn;
-    a.chunks = static_cast<int32_t>(n / 8);
+    a.chunks = static_cast<int32_t>((n + 7) / 8);
     const int lpg = static_cast<int>(block_n / 8);
     // largest unit (chunk slots per lane) that wastes at most 1/16 of the lanes
     int cpl = 1;
@@ -1488,8 +1601,12 @@ extern "C" int pcamd_quant_block(const void* x, int x_dtype, int64_t batch, int6
     // contiguous input, output and scales with whole groups per row: one flat
     // run of chunks, units of two chunks per lane (fastest measured)
     const int64_t gpr = n / block_n;  // groups per row
-    const bool flat = n % block_n == 0 && sxm == n && sym == n && ssn == 1 && ssm == gpr &&
+    const bool flat = fast && n % block_n == 0 && sxm == n && sym == n && ssn == 1 && ssm == gpr &&
                       (batch == 1 || (sxb == m * n && syb == m * n && ssb == m * gpr));
+    if (!fast) {
+      cpl = 2;
+      a.n = n;
+    }
     if (flat) {
       cpl = 2;
       a.total = batch * m * a.chunks;
@@ -1505,7 +1622,7 @@ extern "C" int pcamd_quant_block(const void* x, int x_dtype, int64_t batch, int6
     if (units < UINT32_MAX) return dispatch_dt_fmt<LaunchGroups>(x_dtype, y_dtype, a, lpg, cpl, st);
   }
   const int64_t lpr = block_n / 8;
-  if (fast && block_n >= 32 && lpr <= 64 && (block_m * lpr) % kThreads == 0 &&
+  if (rows && block_n >= 32 && lpr <= 64 && (block_m * lpr) % kThreads == 0 &&
       block_m * lpr / kThreads <= kMaxSlots && batch * mb * nb < UINT32_MAX) {
     TileArgs a{};
     a.x = static_cast<const char*>(x); a.y = static_cast<uint8_t*>(y); a.scale = scale;
@@ -1519,6 +1636,7 @@ extern "C" int pcamd_quant_block(const void* x, int x_dtype, int64_t batch, int6
     a.lpr_shift = 0;
     while ((1 << a.lpr_shift) < a.lpr) ++a.lpr_shift;
     a.fp8_max = fp8_max; a.eps = eps;
+    a.any = !fast;
     // 128 x 128 blocks of 16-bit input: the 1024-thread kernel with 4 H blocks
     // per workgroup when its grid puts at most one workgroup on each CU and
     // fills at least 60 % of them (the whole tensor in flight at once, every
@@ -1528,7 +1646,7 @@ extern "C" int pcamd_quant_block(const void* x, int x_dtype, int64_t batch, int6
     // 256); with more workgroups than CUs (n >= 9216 for H = 2) both were
     // 4-23 % slower, and H = 2 with rows of a multiple of 8 KiB ([8192, 4096])
     // 19 % slower at one workgroup per CU.
-    if (block_m == 128 && block_n == 128 && x_dtype != kF32 && m % 128 == 0 && mb <= 65535 && batch <= 65535 &&
+    if (fast && block_m == 128 && block_n == 128 && x_dtype != kF32 && m % 128 == 0 && mb <= 65535 && batch <= 65535 &&
         n / 512 <= INT32_MAX) {
       const int64_t cus = device_cu_count(st);
       auto fits = [&](int64_t wgs) { return cus > 0 && wgs <= cus && 10 * wgs >= 6 * cus; };
@@ -1644,6 +1762,7 @@ extern "C" int pcamd_quant_channel(const void* x, int x_dtype, int64_t batch, in
   if (!scale) return set_error(PCAMD_ERR_INVALID, "null scale pointer");
   hipStream_t st = static_cast<hipStream_t>(stream);
   const bool fast = row_fast_ok(x, x_dtype, y, n, sxb, sxm, sxn, syb, sym, syn);
+  const bool rows = fast || row_any_ok(n, sxn, syn);
   if (channel_axis == -2 && n == 0) {
     // empty reduction: every row scale is eps / fp8_max (nothing to quantize)
     GenArgs a{};
@@ -1659,19 +1778,20 @@ extern "C" int pcamd_quant_channel(const void* x, int x_dtype, int64_t batch, in
     a.fp8_max = fp8_max; a.eps = eps;
     return dispatch_dt_fmt<LaunchGeneric>(x_dtype, y_dtype, a, 2, st);
   }
-  if (channel_axis == -2 && fast && n / 8 <= 8LL * kThreads && batch * m < INT32_MAX && m < UINT32_MAX) {
+  if (channel_axis == -2 && rows && (n + 7) / 8 <= 8LL * kThreads && batch * m < INT32_MAX && m < UINT32_MAX) {
     RowArgs a{};
     a.x = static_cast<const char*>(x); a.y = static_cast<uint8_t*>(y); a.scale = scale;
     a.m = static_cast<uint32_t>(m); a.sxb = sxb; a.sxm = sxm; a.syb = syb; a.sym = sym;
     a.ssb = ssb; a.ssm = ssc; a.ssn = 0;
-    a.chunks = static_cast<int32_t>(n / 8);
+    a.chunks = static_cast<int32_t>((n + 7) / 8);
+    a.n = fast ? 0 : n;
     a.cpl = static_cast<int32_t>((a.chunks + 63) / 64);  // chunk slots per lane, wave-per-row
     a.segs = 1;
     a.units = static_cast<uint32_t>(batch * m);
     a.fp8_max = fp8_max; a.eps = eps;
     return dispatch_dt_fmt<LaunchRowBlock>(x_dtype, y_dtype, a, st);
   }
-  if (channel_axis == -1 && fast) {
+  if (channel_axis == -1 && rows) {
     ColArgs a{};
     a.x = static_cast<const char*>(x); a.y = static_cast<uint8_t*>(y); a.scale = scale;
     a.m = m; a.n = n; a.sxb = sxb; a.sxm = sxm; a.syb = syb; a.sym = sym;
@@ -1682,10 +1802,10 @@ extern "C" int pcamd_quant_channel(const void* x, int x_dtype, int64_t batch, in
     // Tall tensors: 128-row slabs in parallel (column maxima by atomic max in
     // the scale slots, then a quantize pass). Up to 256 rows one workgroup
     // per strip reads its rows twice.
-    if (m > 256 && a.strips <= INT32_MAX && (m + 127) / 128 <= 65535 && batch <= 65535 &&
+    if ((m > 256 || !fast) && a.strips <= INT32_MAX && (m + 127) / 128 <= 65535 && batch <= 65535 &&
         (batch * n + kThreads - 1) / kThreads <= INT32_MAX)
-      return dispatch_dt_fmt<LaunchColChan>(x_dtype, y_dtype, a, batch, st);
-    return dispatch_dt_fmt<LaunchCols>(x_dtype, y_dtype, a, true, st);
+      return dispatch_dt_fmt<LaunchColChan>(x_dtype, y_dtype, a, batch, !fast, st);
+    if (fast) return dispatch_dt_fmt<LaunchCols>(x_dtype, y_dtype, a, true, st);
   }
   GenArgs a{};
   a.x = static_cast<const char*>(x); a.y = static_cast<uint8_t*>(y); a.scale = scale;
@@ -1714,10 +1834,13 @@ extern "C" int pcamd_quant_tensor(const void* x, int x_dtype, int64_t batch, int
   a.batch = batch; a.m = m; a.n = n; a.sxb = sxb; a.sxm = sxm; a.sxn = sxn;
   a.syb = syb; a.sym = sym; a.syn = syn; a.total = batch * m * n;
   a.fp8_max = fp8_max; a.eps = eps; a.scale_dt = scale_dtype;
-  // one contiguous run of whole chunks in and out
-  const bool flat = row_fast_ok(x, x_dtype, y, n, sxb, sxm, sxn, syb, sym, syn) && sxm == n && sym == n &&
-                    (batch == 1 || (sxb == m * n && syb == m * n)) && (a.total / 8 + 127) / 128 < (1LL << 31);
-  return dispatch_dt_fmt<LaunchTensor>(x_dtype, y_dtype, a, flat, static_cast<hipStream_t>(stream));
+  // one contiguous run of elements in and out, of whole aligned chunks or not
+  const bool fast = row_fast_ok(x, x_dtype, y, n, sxb, sxm, sxn, syb, sym, syn);
+  const bool flat = (fast || row_any_ok(n, sxn, syn)) && (m == 1 || (sxm == n && sym == n)) &&
+                    (batch == 1 || (sxb == m * n && syb == m * n)) && (a.total / 8 + 128) / 128 < (1LL << 31);
+  // (a run of whole chunks may be made of rows that are not)
+  const bool whole = a.total % 8 == 0 && aligned(x, 16) && aligned(y, 8);
+  return dispatch_dt_fmt<LaunchTensor>(x_dtype, y_dtype, a, flat, !whole, static_cast<hipStream_t>(stream));
 }
 
 // plain 16-byte-per-lane streaming copy (measurement of the 1 : 1 ceiling)
