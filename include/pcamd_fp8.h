@@ -43,8 +43,9 @@
 extern "C" {
 #endif
 
-#define PCAMD_ABI_VERSION 4 /* 2: pcamd_bmm_scaled_mixed; 3: pcamd_quant_block_ex, pcamd_quant_block_dual_ex;
-                              4: PCAMD_F64 scale arithmetic of pcamd_quant_tensor */
+#define PCAMD_ABI_VERSION 5 /* 2: pcamd_bmm_scaled_mixed; 3: pcamd_quant_block_ex, pcamd_quant_block_dual_ex;
+                              4: PCAMD_F64 scale arithmetic of pcamd_quant_tensor;
+                              5: pcamd_quant_channel_ws, pcamd_quant_tensor_ws */
 
 /* status codes */
 #define PCAMD_OK 0
@@ -160,6 +161,23 @@ int pcamd_quant_channel(const void *x, int x_dtype, int64_t batch, int64_t m,
                         void *stream);
 
 /*
+ * pcamd_quant_channel with a workspace of pcamd_quant_channel_workspace()
+ * bytes (device memory, 4-byte aligned, contents ignored and overwritten; it
+ * may be NULL, and is not needed where the size is 0). With it the per-column
+ * scales of a tall tensor take two launches instead of four. Same bytes.
+ * Available from PCAMD_ABI_VERSION 5.
+ */
+int64_t pcamd_quant_channel_workspace(int64_t batch, int64_t m, int64_t n,
+                                      int channel_axis);
+int pcamd_quant_channel_ws(const void *x, int x_dtype, int64_t batch,
+                           int64_t m, int64_t n, int64_t sxb, int64_t sxm,
+                           int64_t sxn, void *y, int y_dtype, int64_t syb,
+                           int64_t sym, int64_t syn, float *scale,
+                           int64_t ssb, int64_t ssc, int channel_axis,
+                           float fp8_max, float eps, void *workspace,
+                           int64_t workspace_bytes, void *stream);
+
+/*
  * Per-tensor quantization: amax over the whole tensor, s = max(amax, eps),
  * qs = reciprocal(s) * fp8_max, scale[0] = reciprocal(qs),
  * y = fp8_rne(clamp(x * qs)). quant_scale_out (may be NULL) receives qs. Both
@@ -182,6 +200,21 @@ int pcamd_quant_tensor(const void *x, int x_dtype, int64_t batch, int64_t m,
                        int64_t syn, float *scale, float *quant_scale_out,
                        float fp8_max, float eps, int scale_dtype,
                        void *stream);
+
+/*
+ * pcamd_quant_tensor with a workspace of at least 1024 bytes (device memory,
+ * 16-byte aligned, contents ignored and overwritten; may be NULL): contiguous
+ * tensors then take two launches instead of four. scale_cast (may be NULL)
+ * receives the dequant scale in x's dtype. Same bytes. Available from
+ * PCAMD_ABI_VERSION 5.
+ */
+int pcamd_quant_tensor_ws(const void *x, int x_dtype, int64_t batch,
+                          int64_t m, int64_t n, int64_t sxb, int64_t sxm,
+                          int64_t sxn, void *y, int y_dtype, int64_t syb,
+                          int64_t sym, int64_t syn, float *scale,
+                          float *quant_scale_out, float fp8_max, float eps,
+                          int scale_dtype, void *scale_cast, void *workspace,
+                          int64_t workspace_bytes, void *stream);
 
 /*
  * Scaled FP8 batched GEMM: c[b, m, n] = act(sum_k a[b, m, k] b[b, k, n] *

@@ -42,7 +42,10 @@ EXPORTED_SYMBOLS = (
     "pcamd_quant_block_ex",
     "pcamd_quant_block_dual_ex",
     "pcamd_quant_channel",
+    "pcamd_quant_channel_workspace",
+    "pcamd_quant_channel_ws",
     "pcamd_quant_tensor",
+    "pcamd_quant_tensor_ws",
     "pcamd_bmm_scaled",
     "pcamd_bmm_scaled_mixed",
     "pcamd_bmm_quant_a",
@@ -83,6 +86,12 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.pcamd_quant_channel.argtypes = quant_head + [_ptr, _i64, _i64, _int, _flt, _flt, _ptr]
     lib.pcamd_quant_tensor.restype = _int
     lib.pcamd_quant_tensor.argtypes = quant_head + [_ptr, _ptr, _flt, _flt, _int, _ptr]
+    lib.pcamd_quant_channel_workspace.restype = _i64
+    lib.pcamd_quant_channel_workspace.argtypes = [_i64, _i64, _i64, _int]
+    lib.pcamd_quant_channel_ws.restype = _int
+    lib.pcamd_quant_channel_ws.argtypes = quant_head + [_ptr, _i64, _i64, _int, _flt, _flt, _ptr, _i64, _ptr]
+    lib.pcamd_quant_tensor_ws.restype = _int
+    lib.pcamd_quant_tensor_ws.argtypes = quant_head + [_ptr, _ptr, _flt, _flt, _int, _ptr, _ptr, _i64, _ptr]
     lib.pcamd_bmm_scaled.restype = _int
     lib.pcamd_bmm_scaled.argtypes = (
         [_ptr, _ptr, _int] + [_i64] * 4 + [_i64] * 6 + [_ptr, _int] + [_i64] * 3

@@ -76,9 +76,11 @@ def fp8_quant(
         raise ValueError(f"x must be float32, bfloat16 or float16, got {x.dtype}")
     if quant_dtype not in (torch.float8_e4m3fn, torch.float8_e5m2):
         raise ValueError(f"quant_dtype must be float8_e4m3fn or float8_e5m2, got {quant_dtype}")
-    q, dequant, _ = quant_tensor_raw(x, quant_dtype, eps, fp8_max=float(fp8_range), scale_dtype=x.dtype)
-    # the scale steps were rounded to x's dtype on the GPU, so this cast is exact
-    return q, dequant.to(x.dtype)
+    # the scale steps are rounded to x's dtype on the GPU, so its cast to that dtype is exact
+    reciprocal = torch.empty((), dtype=x.dtype, device=x.device)
+    q, _, _ = quant_tensor_raw(x, quant_dtype, eps, fp8_max=float(fp8_range), scale_dtype=x.dtype,
+                               scale_cast=reciprocal)
+    return q, reciprocal
 
 
 def fp8_bmm_quant(

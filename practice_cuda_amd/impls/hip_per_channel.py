@@ -58,13 +58,18 @@ def hip_per_channel_quant(
     scale_storage = torch.empty((batch, channels), device=x.device, dtype=torch.float32)
 
     L = _lib.lib()
+    # column maxima of the two-launch form (tall tensors); the caller's stream orders its reuse
+    ws, ws_bytes = None, 0
+    if channel_axis == -1 and m > 256:
+        ws_bytes = L.pcamd_quant_channel_workspace(batch, m, n, channel_axis)
+        ws = torch.empty(ws_bytes, device=x.device, dtype=torch.uint8)
     with torch.cuda.device(x.device):
-        rc = L.pcamd_quant_channel(
+        rc = L.pcamd_quant_channel_ws(
             _lib.ptr(x), _lib.dtype_code(x.dtype), batch, m, n, *xs,
             _lib.ptr(output), _lib.dtype_code(fp8_dtype), *ys,
             _lib.ptr(scale_storage), *scale_storage.stride(), channel_axis,
-            float(torch.finfo(fp8_dtype).max), float(eps), _lib.stream_of(x))
-    _lib.check(rc, "pcamd_quant_channel")
+            float(torch.finfo(fp8_dtype).max), float(eps), _lib.ptr(ws), ws_bytes, _lib.stream_of(x))
+    _lib.check(rc, "pcamd_quant_channel_ws")
 
     dequant_scale = scale_storage.squeeze(0) if x.ndim == 2 else scale_storage
     return QuantResult(

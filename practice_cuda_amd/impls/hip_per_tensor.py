@@ -18,8 +18,12 @@ from ..registry import QuantResult, register_bmm, register_quant
 from . import _common as C
 
 
+_WORKSPACE_FLOATS = 256  # pcamd_quant_tensor_ws: 1024 bytes
+
+
 def quant_tensor_raw(x: torch.Tensor, fp8_dtype: torch.dtype, eps: float, *,
-                     fp8_max: float | None = None, scale_dtype: torch.dtype = torch.float32):
+                     fp8_max: float | None = None, scale_dtype: torch.dtype = torch.float32,
+                     scale_cast: torch.Tensor | None = None):
     """Launch the per-tensor kernels; returns (fp8 tensor, dequant scale, quant scale).
 
     scale_dtype is the dtype the scalar scale steps are rounded to (fp32 for
@@ -28,21 +32,25 @@ def quant_tensor_raw(x: torch.Tensor, fp8_dtype: torch.dtype, eps: float, *,
     modules/float8/float8_utils.py:45-48: qs = fp32(fp8_max / max(fp64(amax),
     eps)), dequant = its fp32 reciprocal), which the reference's training
     layer quantizes with. fp8_max defaults to the fp8 format's largest finite
-    value.
+    value. scale_cast: a 0-d tensor of x's dtype that receives the dequant
+    scale as well.
     """
     output = torch.empty_like(x, dtype=fp8_dtype, memory_format=torch.preserve_format)
     batch, m, n, xs, ys = C.dims3(x, output)
-    scales = torch.empty(2, device=x.device, dtype=torch.float32)
+    # the two scales, and (16-byte aligned) the kernels' workspace
+    scales = torch.empty(4 + _WORKSPACE_FLOATS, device=x.device, dtype=torch.float32)
     L = _lib.lib()
     _lib.require_gpu_tensor(x, "x")
     with torch.cuda.device(x.device):
-        rc = L.pcamd_quant_tensor(
+        base = scales.data_ptr()
+        rc = L.pcamd_quant_tensor_ws(
             _lib.ptr(x), _lib.dtype_code(x.dtype), batch, m, n, *xs,
             _lib.ptr(output), _lib.dtype_code(fp8_dtype), *ys,
-            _lib.ptr(scales[0:1]), _lib.ptr(scales[1:2]),
+            base, base + 4,
             float(torch.finfo(fp8_dtype).max if fp8_max is None else fp8_max), float(eps),
-            _lib.F64 if scale_dtype == torch.float64 else _lib.dtype_code(scale_dtype), _lib.stream_of(x))
-    _lib.check(rc, "pcamd_quant_tensor")
+            _lib.F64 if scale_dtype == torch.float64 else _lib.dtype_code(scale_dtype),
+            _lib.ptr(scale_cast), base + 16, 4 * _WORKSPACE_FLOATS, _lib.stream_of(x))
+    _lib.check(rc, "pcamd_quant_tensor_ws")
     return output, scales[0], scales[1]
 
 
