@@ -140,13 +140,29 @@ def dtype_code(dtype: torch.dtype) -> int:
         raise ValueError(f"unsupported dtype for the HIP path: {dtype}") from exc
 
 
-def stream_of(t: torch.Tensor) -> ctypes.c_void_p:
+def stream_of(t: torch.Tensor) -> int:
     """hipStream_t of torch's current stream on the tensor's device."""
-    return ctypes.c_void_p(torch.cuda.current_stream(t.device).cuda_stream)
+    return torch._C._cuda_getCurrentRawStream(t.get_device())
 
 
-def ptr(t) -> ctypes.c_void_p:
-    return ctypes.c_void_p(0 if t is None else t.data_ptr())
+def ptr(t) -> int:
+    return 0 if t is None else t.data_ptr()
+
+
+def launch(fn, t: torch.Tensor, *args) -> int:
+    """fn(*args, stream) with t's device current and torch's current stream on
+    it; returns the status. The device is switched only when it is another
+    one: the switch and its objects cost 1.3 us, the raw stream 0.1 us (the
+    stream object 2.1 us) of a call's host time."""
+    index = t.get_device()
+    if torch._C._cuda_getDevice() == index:
+        return fn(*args, torch._C._cuda_getCurrentRawStream(index))
+    with torch.cuda.device(index):
+        return fn(*args, torch._C._cuda_getCurrentRawStream(index))
+
+
+# largest finite value per fp8 type
+FP8_MAX = {t: float(torch.finfo(t).max) for t in (torch.float8_e4m3fn, torch.float8_e5m2)}
 
 
 def check(status: int, what: str) -> None:

@@ -206,17 +206,16 @@ def launch_bmm(a_tensor, b_tensor, out, bias, bias_strides, bias_code, sa, sa_st
     fmt = ((_lib.dtype_code(a_tensor.dtype),) if a_tensor.dtype == b_tensor.dtype
            else (_lib.dtype_code(a_tensor.dtype), _lib.dtype_code(b_tensor.dtype)))
     entry = L.pcamd_bmm_scaled if len(fmt) == 1 else L.pcamd_bmm_scaled_mixed
-    with torch.cuda.device(a_tensor.device):
-        rc = entry(
-            *((_lib.ptr(a_tensor), _lib.ptr(b_tensor), fmt[0]) if len(fmt) == 1
-              else (_lib.ptr(a_tensor), fmt[0], _lib.ptr(b_tensor), fmt[1])),
-            batch, m, n, k,
-            *a_tensor.stride(), *b_tensor.stride(),
-            _lib.ptr(out), _lib.dtype_code(out.dtype), *out.stride(),
-            _lib.ptr(bias), bias_code, *bias_strides,
-            _lib.ptr(sa), *sa_strides, _lib.ptr(sb), *sb_strides,
-            scale_mode, int(scales_are_quant), qbm, qbk, qbn,
-            _lib.ACT_GELU if activation == "gelu" else _lib.ACT_NONE,
-            _lib.stream_of(a_tensor))
+    rc = _lib.launch(
+        entry, a_tensor,
+        *((a_tensor.data_ptr(), b_tensor.data_ptr(), fmt[0]) if len(fmt) == 1
+          else (a_tensor.data_ptr(), fmt[0], b_tensor.data_ptr(), fmt[1])),
+        batch, m, n, k,
+        *a_tensor.stride(), *b_tensor.stride(),
+        out.data_ptr(), _lib.dtype_code(out.dtype), *out.stride(),
+        _lib.ptr(bias), bias_code, *bias_strides,
+        sa.data_ptr(), *sa_strides, _lib.ptr(sb), *sb_strides,
+        scale_mode, int(scales_are_quant), qbm, qbk, qbn,
+        _lib.ACT_GELU if activation == "gelu" else _lib.ACT_NONE)
     _lib.check(rc, "pcamd_bmm_scaled" if len(fmt) == 1 else "pcamd_bmm_scaled_mixed")
     return out

@@ -54,19 +54,18 @@ def hip_per_block_quant(
     batch, m, n, xs, ys = C.dims3(x, output)
     m_blocks = -(-m // block_m)
     n_blocks = -(-n // block_n)
-    scale_storage = torch.empty((batch, m_blocks, n_blocks), device=x.device, dtype=torch.float32)
+    dequant_scale = torch.empty((m_blocks, n_blocks) if x.ndim == 2 else (batch, m_blocks, n_blocks),
+                                device=x.device, dtype=torch.float32)
 
-    L = _lib.lib()
-    with torch.cuda.device(x.device):
-        rc = L.pcamd_quant_block_ex(
-            _lib.ptr(x), _lib.dtype_code(x.dtype), batch, m, n, *xs,
-            _lib.ptr(output), _lib.dtype_code(fp8_dtype), *ys,
-            _lib.ptr(scale_storage), *scale_storage.stride(),
-            block_m, block_n, float(torch.finfo(fp8_dtype).max), float(eps),
-            _lib.QUANT_CACHED_OUTPUT if cache_outputs else 0, _lib.stream_of(x))
+    rc = _lib.launch(
+        _lib.lib().pcamd_quant_block_ex, x,
+        x.data_ptr(), _lib.dtype_code(x.dtype), batch, m, n, *xs,
+        output.data_ptr(), _lib.dtype_code(fp8_dtype), *ys,
+        dequant_scale.data_ptr(), m_blocks * n_blocks, n_blocks, 1,
+        block_m, block_n, _lib.FP8_MAX[fp8_dtype], float(eps),
+        _lib.QUANT_CACHED_OUTPUT if cache_outputs else 0)
     _lib.check(rc, "pcamd_quant_block")
 
-    dequant_scale = scale_storage.squeeze(0) if x.ndim == 2 else scale_storage
     return QuantResult(
         tensor=output,
         dequant_scale=dequant_scale,
@@ -112,30 +111,33 @@ def hip_per_block_quant_dual(
 
     out_row = torch.empty_like(x, dtype=fp8_dtype, memory_format=torch.preserve_format)
     if col_transposed:
-        pitch = -(-x.shape[-2] // 16) * 16
-        out_col = torch.empty(*x.shape[:-2], x.shape[-1], pitch, dtype=fp8_dtype,
-                              device=x.device)[..., :x.shape[-2]].transpose(-1, -2)
+        rows, cols = x.shape[-2:]
+        pitch = -(-rows // 16) * 16
+        # a [.., N, pitch] buffer seen as [.., M, N]: one allocation, no slice and transpose views
+        out_col = torch.empty_strided(x.shape, (cols * pitch, 1, pitch) if x.ndim == 3 else (1, pitch),
+                                      dtype=fp8_dtype, device=x.device)
     else:
         out_col = torch.empty_strided(out_row.shape, out_row.stride(), dtype=fp8_dtype, device=x.device)
     batch, m, n, xs, ys = C.dims3(x, out_row)
     yc = (0, *out_col.stride()) if out_col.ndim == 2 else tuple(out_col.stride())
-    s_row = torch.empty((batch, m, -(-n // block)), device=x.device, dtype=torch.float32)
-    s_col = torch.empty((batch, -(-m // block), n), device=x.device, dtype=torch.float32)
+    nb, mb = -(-n // block), -(-m // block)
+    lead = (batch,) if x.ndim == 3 else ()
+    s_row = torch.empty((*lead, m, nb), device=x.device, dtype=torch.float32)
+    s_col = torch.empty((*lead, mb, n), device=x.device, dtype=torch.float32)
 
-    L = _lib.lib()
-    with torch.cuda.device(x.device):
-        rc = L.pcamd_quant_block_dual_ex(
-            _lib.ptr(x), _lib.dtype_code(x.dtype), batch, m, n, *xs,
-            _lib.ptr(out_row), *ys, _lib.ptr(out_col), *yc, _lib.dtype_code(fp8_dtype),
-            _lib.ptr(s_row), *s_row.stride(), _lib.ptr(s_col), *s_col.stride(),
-            block, float(torch.finfo(fp8_dtype).max), float(eps),
-            _lib.QUANT_CACHED_OUTPUT if cache_outputs else 0, _lib.stream_of(x))
+    rc = _lib.launch(
+        _lib.lib().pcamd_quant_block_dual_ex, x,
+        x.data_ptr(), _lib.dtype_code(x.dtype), batch, m, n, *xs,
+        out_row.data_ptr(), *ys, out_col.data_ptr(), *yc, _lib.dtype_code(fp8_dtype),
+        s_row.data_ptr(), m * nb, nb, 1, s_col.data_ptr(), mb * n, n, 1,
+        block, _lib.FP8_MAX[fp8_dtype], float(eps),
+        _lib.QUANT_CACHED_OUTPUT if cache_outputs else 0)
     _lib.check(rc, "pcamd_quant_block_dual")
 
     def result(q, s, bm, bn):
         return QuantResult(
             tensor=q,
-            dequant_scale=s.squeeze(0) if x.ndim == 2 else s,
+            dequant_scale=s,
             impl="hip_per_block",
             granularity="block",
             meta={"logical_shape": tuple(x.shape), "fp8_dtype": str(fp8_dtype), "block_m": bm, "block_n": bn},
@@ -293,17 +295,17 @@ def hip_per_block_bmm_quant_a(
     rc = _lib.ERR_UNSUPPORTED
     fused = always_fused or fused_streams(n, k, qbn)
     if in_b in ("n-major", "k-major") and x3.stride(-1) == 1 and fused:
-        with torch.cuda.device(x3.device):
-            rc = L.pcamd_bmm_quant_a(
-                _lib.ptr(x3), _lib.dtype_code(x3.dtype), _lib.ptr(b.tensor), _lib.dtype_code(fp8_dtype),
-                batch, m, n, k, *x3.stride(), *b.tensor.stride(),
-                _lib.ptr(out), _lib.dtype_code(out.dtype), *out.stride(),
-                _lib.ptr(bias), bias_code, *bias_strides,
-                _lib.ptr(b.dequant_scale), *b.dequant_scale.stride(), qbn,
-                _lib.ptr(qa), *(qa.stride() if qa is not None else (0, 0, 0)),
-                _lib.ptr(sa), *(sa.stride() if sa is not None else (0, 0, 0)),
-                float(torch.finfo(fp8_dtype).max), float(eps),
-                _lib.ACT_GELU if activation == "gelu" else _lib.ACT_NONE, _lib.stream_of(x3))
+        rc = _lib.launch(
+            L.pcamd_bmm_quant_a, x3,
+            _lib.ptr(x3), _lib.dtype_code(x3.dtype), _lib.ptr(b.tensor), _lib.dtype_code(fp8_dtype),
+            batch, m, n, k, *x3.stride(), *b.tensor.stride(),
+            _lib.ptr(out), _lib.dtype_code(out.dtype), *out.stride(),
+            _lib.ptr(bias), bias_code, *bias_strides,
+            _lib.ptr(b.dequant_scale), *b.dequant_scale.stride(), qbn,
+            _lib.ptr(qa), *(qa.stride() if qa is not None else (0, 0, 0)),
+            _lib.ptr(sa), *(sa.stride() if sa is not None else (0, 0, 0)),
+            float(torch.finfo(fp8_dtype).max), float(eps),
+            _lib.ACT_GELU if activation == "gelu" else _lib.ACT_NONE)
     if rc == _lib.ERR_UNSUPPORTED:
         qres = hip_per_block_quant(x3, block_m=1, block_n=128, fp8_dtype=fp8_dtype, eps=eps)
         hip_per_block_bmm(qres, b, out_dtype=out_dtype, bias=bias, out=out, activation=activation)

@@ -55,7 +55,8 @@ def hip_per_channel_quant(
     C.matrix_layout(output, "quant output")
     batch, m, n, xs, ys = C.dims3(x, output)
     channels = m if channel_axis == -2 else n
-    scale_storage = torch.empty((batch, channels), device=x.device, dtype=torch.float32)
+    dequant_scale = torch.empty((channels,) if x.ndim == 2 else (batch, channels), device=x.device,
+                                dtype=torch.float32)
 
     L = _lib.lib()
     # column maxima of the two-launch form (tall tensors); the caller's stream orders its reuse
@@ -63,15 +64,14 @@ def hip_per_channel_quant(
     if channel_axis == -1 and m > 256:
         ws_bytes = L.pcamd_quant_channel_workspace(batch, m, n, channel_axis)
         ws = torch.empty(ws_bytes, device=x.device, dtype=torch.uint8)
-    with torch.cuda.device(x.device):
-        rc = L.pcamd_quant_channel_ws(
-            _lib.ptr(x), _lib.dtype_code(x.dtype), batch, m, n, *xs,
-            _lib.ptr(output), _lib.dtype_code(fp8_dtype), *ys,
-            _lib.ptr(scale_storage), *scale_storage.stride(), channel_axis,
-            float(torch.finfo(fp8_dtype).max), float(eps), _lib.ptr(ws), ws_bytes, _lib.stream_of(x))
+    rc = _lib.launch(
+        L.pcamd_quant_channel_ws, x,
+        x.data_ptr(), _lib.dtype_code(x.dtype), batch, m, n, *xs,
+        output.data_ptr(), _lib.dtype_code(fp8_dtype), *ys,
+        dequant_scale.data_ptr(), channels, 1, channel_axis,
+        _lib.FP8_MAX[fp8_dtype], float(eps), _lib.ptr(ws), ws_bytes)
     _lib.check(rc, "pcamd_quant_channel_ws")
 
-    dequant_scale = scale_storage.squeeze(0) if x.ndim == 2 else scale_storage
     return QuantResult(
         tensor=output,
         dequant_scale=dequant_scale,

@@ -41,15 +41,15 @@ def quant_tensor_raw(x: torch.Tensor, fp8_dtype: torch.dtype, eps: float, *,
     scales = torch.empty(4 + _WORKSPACE_FLOATS, device=x.device, dtype=torch.float32)
     L = _lib.lib()
     _lib.require_gpu_tensor(x, "x")
-    with torch.cuda.device(x.device):
-        base = scales.data_ptr()
-        rc = L.pcamd_quant_tensor_ws(
-            _lib.ptr(x), _lib.dtype_code(x.dtype), batch, m, n, *xs,
-            _lib.ptr(output), _lib.dtype_code(fp8_dtype), *ys,
-            base, base + 4,
-            float(torch.finfo(fp8_dtype).max if fp8_max is None else fp8_max), float(eps),
-            _lib.F64 if scale_dtype == torch.float64 else _lib.dtype_code(scale_dtype),
-            _lib.ptr(scale_cast), base + 16, 4 * _WORKSPACE_FLOATS, _lib.stream_of(x))
+    base = scales.data_ptr()
+    rc = _lib.launch(
+        L.pcamd_quant_tensor_ws, x,
+        x.data_ptr(), _lib.dtype_code(x.dtype), batch, m, n, *xs,
+        output.data_ptr(), _lib.dtype_code(fp8_dtype), *ys,
+        base, base + 4,
+        float(torch.finfo(fp8_dtype).max if fp8_max is None else fp8_max), float(eps),
+        _lib.F64 if scale_dtype == torch.float64 else _lib.dtype_code(scale_dtype),
+        _lib.ptr(scale_cast), base + 16, 4 * _WORKSPACE_FLOATS)
     _lib.check(rc, "pcamd_quant_tensor_ws")
     return output, scales[0], scales[1]
 

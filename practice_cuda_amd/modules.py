@@ -46,8 +46,7 @@ _FP8 = (torch.float8_e4m3fn, torch.float8_e5m2)
 # ---------------------------------------------------------------------------
 # custom ops
 # ---------------------------------------------------------------------------
-@torch.library.custom_op("pcamd::block_scaled_bmm", mutates_args=())
-def block_scaled_bmm(
+def _block_scaled_bmm(
     a: torch.Tensor,
     sa: torch.Tensor,
     b: torch.Tensor,
@@ -95,13 +94,15 @@ def block_scaled_bmm(
                         _lib.SCALE_BLOCK, False, qbm, qbk, qbn, "none", batch, m, n, k)
 
 
+block_scaled_bmm = torch.library.custom_op("pcamd::block_scaled_bmm", mutates_args=())(_block_scaled_bmm)
+
+
 @block_scaled_bmm.register_fake
 def _(a, sa, b, sb, bias, qbm, qbk, qbn, out_dtype):
     return a.new_empty((a.shape[0], a.shape[1], b.shape[2]), dtype=out_dtype)
 
 
-@torch.library.custom_op("pcamd::tensor_scaled_bmm", mutates_args=())
-def tensor_scaled_bmm(a: torch.Tensor, b: torch.Tensor, scale: torch.Tensor, bias: Optional[torch.Tensor],
+def _tensor_scaled_bmm(a: torch.Tensor, b: torch.Tensor, scale: torch.Tensor, bias: Optional[torch.Tensor],
                       out_dtype: torch.dtype) -> torch.Tensor:
     """``C[b] = (A[b] @ B[b]) * scale (+ bias[b] over M)``; scale: fp32, one element."""
     batch, m, k = a.shape
@@ -119,19 +120,24 @@ def tensor_scaled_bmm(a: torch.Tensor, b: torch.Tensor, scale: torch.Tensor, bia
                         _lib.SCALE_TENSOR, False, 1, 128, 1, "none", batch, m, n, k)
 
 
+tensor_scaled_bmm = torch.library.custom_op("pcamd::tensor_scaled_bmm", mutates_args=())(_tensor_scaled_bmm)
+
+
 @tensor_scaled_bmm.register_fake
 def _(a, b, scale, bias, out_dtype):
     return a.new_empty((a.shape[0], a.shape[1], b.shape[2]), dtype=out_dtype)
 
 
-@torch.library.custom_op("pcamd::quant_block", mutates_args=())
-def quant_block(x: torch.Tensor, block_m: int, block_n: int, fp8_dtype: torch.dtype,
+def _quant_block(x: torch.Tensor, block_m: int, block_n: int, fp8_dtype: torch.dtype,
                 eps: float) -> tuple[torch.Tensor, torch.Tensor]:
     """(fp8 [B,M,N], fp32 dequant scales [B, ceil(M/block_m), ceil(N/block_n)]),
     written with cache-allocating stores: the layer's GEMM reads them next."""
     q = hip_per_block_quant(x, block_m=block_m, block_n=block_n, fp8_dtype=fp8_dtype, eps=eps,
                             cache_outputs=True)
     return q.tensor, q.dequant_scale
+
+
+quant_block = torch.library.custom_op("pcamd::quant_block", mutates_args=())(_quant_block)
 
 
 @quant_block.register_fake
@@ -141,8 +147,7 @@ def _(x, block_m, block_n, fp8_dtype, eps):
             x.new_empty((b, -(-m // block_m), -(-n // block_n)), dtype=torch.float32))
 
 
-@torch.library.custom_op("pcamd::quant_block_dual", mutates_args=())
-def quant_block_dual(x: torch.Tensor, block: int, fp8_dtype: torch.dtype,
+def _quant_block_dual(x: torch.Tensor, block: int, fp8_dtype: torch.dtype,
                      eps: float) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor]:
     """``quant_block(x, 1, block)`` and ``quant_block(x, block, 1)`` from one read
     of x: (fp8 1 x block, its scales [B, M, ceil(N/block)], fp8 block x 1 stored
@@ -154,6 +159,9 @@ def quant_block_dual(x: torch.Tensor, block: int, fp8_dtype: torch.dtype,
     return r.tensor, r.dequant_scale, c.tensor, c.dequant_scale
 
 
+quant_block_dual = torch.library.custom_op("pcamd::quant_block_dual", mutates_args=())(_quant_block_dual)
+
+
 @quant_block_dual.register_fake
 def _(x, block, fp8_dtype, eps):
     b, m, n = x.shape
@@ -162,17 +170,47 @@ def _(x, block, fp8_dtype, eps):
             x.new_empty((b, -(-m // block), n), dtype=torch.float32))
 
 
-@torch.library.custom_op("pcamd::quant_tensor", mutates_args=())
-def quant_tensor(x: torch.Tensor, fp8_dtype: torch.dtype, eps: float) -> tuple[torch.Tensor, torch.Tensor]:
+def _quant_tensor(x: torch.Tensor, fp8_dtype: torch.dtype, eps: float) -> tuple[torch.Tensor, torch.Tensor]:
     """(fp8 tensor like x, fp32 dequant scale of shape [1]) with torchao's
     tensorwise scale (the division in fp64, rounded once to fp32)."""
     q, dequant, _ = quant_tensor_raw(x, fp8_dtype, eps, scale_dtype=torch.float64)
     return q, dequant.reshape(1).clone()
 
 
+quant_tensor = torch.library.custom_op("pcamd::quant_tensor", mutates_args=())(_quant_tensor)
+
+
 @quant_tensor.register_fake
 def _(x, fp8_dtype, eps):
     return torch.empty_like(x, dtype=fp8_dtype), x.new_empty((1,), dtype=torch.float32)
+
+
+class _Direct:
+    """The ops' own functions, without the dispatcher around them."""
+
+    block_scaled_bmm = staticmethod(_block_scaled_bmm)
+    tensor_scaled_bmm = staticmethod(_tensor_scaled_bmm)
+    quant_block = staticmethod(_quant_block)
+    quant_block_dual = staticmethod(_quant_block_dual)
+    quant_tensor = staticmethod(_quant_tensor)
+
+
+_PLAIN = (torch.Tensor, nn.Parameter)
+
+
+def _ops(*tensors):
+    """What the layer calls: ``torch.ops.pcamd`` wherever something may look at
+    or stand in for the ops (compilation, a dispatch mode such as a tracer, a
+    counter or selective checkpointing, a function transform, a tensor
+    subclass), else the functions they run, which spares eager steps the
+    dispatcher's Python layers (6.5 us of host time per op, six ops per step).
+    Either way the same launches on the same stream; only called where autograd
+    does not record (inside the autograd function)."""
+    if (torch.compiler.is_compiling() or torch._C._len_torch_dispatch_stack() or torch.is_grad_enabled()
+            or torch._C._functorch.peek_interpreter_stack() is not None
+            or any(t is not None and type(t) not in _PLAIN for t in tensors)):
+        return torch.ops.pcamd
+    return _Direct
 
 
 # ---------------------------------------------------------------------------
@@ -210,8 +248,8 @@ class Float8BlockBMMLinearConfig:
             raise ValueError("the block recipe uses 128-wide quant blocks")
 
 
-def _block_gemm(qa, sa, qb, sb, bias, qbm, qbn, out_dtype, block):
-    return torch.ops.pcamd.block_scaled_bmm(qa, sa, qb, sb, bias, qbm, block, qbn, out_dtype)
+def _block_gemm(ops, qa, sa, qb, sb, bias, qbm, qbn, out_dtype, block):
+    return ops.block_scaled_bmm(qa, sa, qb, sb, bias, qbm, block, qbn, out_dtype)
 
 
 class _Float8BlockBMMLinearFunction(torch.autograd.Function):
@@ -221,24 +259,25 @@ class _Float8BlockBMMLinearFunction(torch.autograd.Function):
     def forward(ctx, input: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor],
                 config: Float8BlockBMMLinearConfig) -> torch.Tensor:
         f8, eps, blk = config.fp8_dtype, config.eps, config.block
+        ops = _ops(input, weight)
         ctx.config = config
         ctx.has_bias = bias is not None
         bias_k = None if bias is None else bias.to(input.dtype)
         if config.granularity == "tensor":
-            qx, sx = torch.ops.pcamd.quant_tensor(input, f8, eps)
-            qw, sw = torch.ops.pcamd.quant_tensor(weight, f8, eps)
+            qx, sx = ops.quant_tensor(input, f8, eps)
+            qw, sw = ops.quant_tensor(weight, f8, eps)
             ctx.save_for_backward(qx, sx, qw, sw)
-            return torch.ops.pcamd.tensor_scaled_bmm(qx, qw.transpose(-2, -1), sx * sw, bias_k, input.dtype)
+            return ops.tensor_scaled_bmm(qx, qw.transpose(-2, -1), sx * sw, bias_k, input.dtype)
         if ctx.needs_input_grad[1]:
             # wgrad needs X quantized in 128-row blocks too: both from one read
-            qx, sx, qxm, sxm = torch.ops.pcamd.quant_block_dual(input, blk, f8, eps)
+            qx, sx, qxm, sxm = ops.quant_block_dual(input, blk, f8, eps)
         else:
-            qx, sx = torch.ops.pcamd.quant_block(input, 1, blk, f8, eps)  # [B,M,K], [B,M,K/128]
+            qx, sx = ops.quant_block(input, 1, blk, f8, eps)  # [B,M,K], [B,M,K/128]
             qxm = sxm = None
-        qw, sw = torch.ops.pcamd.quant_block(weight, blk, blk, f8, eps)   # [B,N,K], [B,N/128,K/128]
+        qw, sw = ops.quant_block(weight, blk, blk, f8, eps)   # [B,N,K], [B,N/128,K/128]
         ctx.save_for_backward(qxm, sxm, qw, sw)
         # B = W^T: [B,K,N] contiguous along K; its scales [B,K/128,N/128]
-        return _block_gemm(qx, sx, qw.transpose(-2, -1), sw.transpose(-2, -1), bias_k, 1, blk, input.dtype, blk)
+        return _block_gemm(ops, qx, sx, qw.transpose(-2, -1), sw.transpose(-2, -1), bias_k, 1, blk, input.dtype, blk)
 
     @staticmethod
     def backward(ctx, grad_output: torch.Tensor):
@@ -246,31 +285,33 @@ class _Float8BlockBMMLinearFunction(torch.autograd.Function):
         eps, blk = config.eps, config.block
         f8 = config.grad_fp8_dtype or config.fp8_dtype  # dY's format
         dy = grad_output.contiguous()
+        saved = ctx.saved_tensors  # once: each access runs the saved-tensor hooks
+        ops = _ops(dy, *saved)
         grad_input = grad_weight = grad_bias = None
         if config.granularity == "tensor":
-            qx, sx, qw, sw = ctx.saved_tensors
-            qdy, sdy = torch.ops.pcamd.quant_tensor(dy, f8, eps)
+            qx, sx, qw, sw = saved
+            qdy, sdy = ops.quant_tensor(dy, f8, eps)
             if ctx.needs_input_grad[0]:
-                grad_input = torch.ops.pcamd.tensor_scaled_bmm(qdy, qw, sdy * sw, None, dy.dtype)
+                grad_input = ops.tensor_scaled_bmm(qdy, qw, sdy * sw, None, dy.dtype)
             if ctx.needs_input_grad[1]:
-                grad_weight = torch.ops.pcamd.tensor_scaled_bmm(qdy.transpose(-2, -1), qx, sdy * sx, None, dy.dtype)
+                grad_weight = ops.tensor_scaled_bmm(qdy.transpose(-2, -1), qx, sdy * sx, None, dy.dtype)
         else:
-            qxm, sxm, qw, sw = ctx.saved_tensors
+            qxm, sxm, qw, sw = saved
             need_dx, need_dw = ctx.needs_input_grad[0], ctx.needs_input_grad[1]
             if need_dx and need_dw:
                 # dY quantized 1x128 along N (dgrad) and in 128-row blocks (wgrad) from one read
-                qdy, sdy, qdt, sdt = torch.ops.pcamd.quant_block_dual(dy, blk, f8, eps)
+                qdy, sdy, qdt, sdt = ops.quant_block_dual(dy, blk, f8, eps)
             elif need_dx:
-                qdy, sdy = torch.ops.pcamd.quant_block(dy, 1, blk, f8, eps)      # [B,M,N], [B,M,N/128]
+                qdy, sdy = ops.quant_block(dy, 1, blk, f8, eps)      # [B,M,N], [B,M,N/128]
             elif need_dw:
-                qdt, sdt = torch.ops.pcamd.quant_block(dy, blk, 1, f8, eps)      # [B,M,N], [B,M/128,N]
+                qdt, sdt = ops.quant_block(dy, blk, 1, f8, eps)      # [B,M,N], [B,M/128,N]
             if need_dx:
                 # dX = dY W: A = dY [B,M,N] 1x128 along N; B = W [B,N,K] (N = reduction)
-                grad_input = _block_gemm(qdy, sdy, qw, sw, None, 1, blk, dy.dtype, blk)
+                grad_input = _block_gemm(ops, qdy, sdy, qw, sw, None, 1, blk, dy.dtype, blk)
             if need_dw:
                 # dW = dY^T X: dY and X (quantized in forward) in 128-row blocks along M; from
                 # quant_block_dual both are stored transposed, so A = dY^T and B = X are K-major
-                grad_weight = _block_gemm(qdt.transpose(-2, -1), sdt.transpose(-2, -1), qxm, sxm, None,
+                grad_weight = _block_gemm(ops, qdt.transpose(-2, -1), sdt.transpose(-2, -1), qxm, sxm, None,
                                           1, 1, dy.dtype, blk)
         if ctx.has_bias and ctx.needs_input_grad[2]:
             grad_bias = dy.sum(dim=1)

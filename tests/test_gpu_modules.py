@@ -195,3 +195,40 @@ def test_config5_shape_within_fp8_error(dev):
     assert rel(y, torch.matmul(x.float(), w.transpose(-1, -2).contiguous())) < 0.05
     assert rel(dx, torch.matmul(dy.float(), w)) < 0.05
     assert rel(dw, torch.matmul(dy.float().transpose(-1, -2).contiguous(), x.float())) < 0.05
+
+
+def test_layer_ops_seen_by_dispatch_modes(dev):
+    """Under a dispatch mode the layer's launches go through torch.ops.pcamd,
+    where the mode sees them; without one it calls their functions. Same bits,
+    and saved-tensor hooks run once per saved tensor either way."""
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    class Names(TorchDispatchMode):
+        def __init__(self):
+            super().__init__()
+            self.names = []
+
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            self.names.append(str(func))
+            return func(*args, **(kwargs or {}))
+
+    torch.manual_seed(0)
+    layer = Float8BMMLinear(1, 256, 384, device=dev, dtype=torch.bfloat16)
+    x = torch.randn(1, 200, 256, device=dev, dtype=torch.bfloat16, requires_grad=True)
+    dy = torch.randn(1, 200, 384, device=dev, dtype=torch.bfloat16)
+
+    def step():
+        y = layer(x)
+        return [y.detach(), *torch.autograd.grad(y, [x, layer.weight, layer.bias], dy)]
+
+    plain = step()
+    with Names() as mode:
+        seen = step()
+    assert sum("pcamd.block_scaled_bmm" in n for n in mode.names) == 3
+    assert sum("pcamd.quant_block_dual" in n for n in mode.names) == 2
+    assert all(torch.equal(a, b) for a, b in zip(plain, seen))
+    unpacked = []
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t, lambda t: unpacked.append(1) or t):
+        hooked = step()
+    assert len(unpacked) == 4
+    assert all(torch.equal(a, b) for a, b in zip(plain, hooked))
