@@ -41,6 +41,8 @@ SETTLE_MS = 100.0            # untimed load before the first (headline) measurem
 CONFIG4_KERNEL = "pcamd::bmms::bmm_stream_kernel<3>"
 # template arguments: A K-major, B K-major, A / B fp8 formats, scale mode, B-scale kind,
 # sub-tiles per wave, ragged K, transposed output (wgrad: 256 x 224 tiles of C^T)
+# (as profiled; the kernel has since gained a tenth argument, false for these
+# instantiations, whose code is unchanged)
 CONFIG5_KERNELS = {"fwd_a_k_b_k": ("fwd", ["pcamd::bmmw::bmm_wide_kernel<true, true, 3, 3, 0, 0, 8, false, false>"]),
                    "dgrad_a_k_b_n": ("dgrad",
                                      ["pcamd::bmmw::bmm_wide_kernel<true, false, 3, 3, 0, 0, 8, false, false>"]),

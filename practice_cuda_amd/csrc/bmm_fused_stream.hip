@@ -107,9 +107,9 @@ __global__ __launch_bounds__(NT, 1) void bmm_fused_stream_kernel(FastArgs a) {
   // B: global -> LDS one step ahead (inline asm, ordered by hand); K block
   // kb lands in LDS slot kb % (2 G)
   const v4i rsb = lds::make_rsrc(a.b + bidx * a.sbb, a.b_extent);
-  using LB = typename std::conditional<B_K, bmmw::KMajorLoader<BCOLS>, lds::MNMajorLoader<256, WAVES>>::type;
+  using LB = typename std::conditional<B_K, bmmw::KMajorLoader<BCOLS, WAVES>, lds::MNMajorLoader<256, WAVES>>::type;
   const LB load_b = [&] {
-    if constexpr (B_K) return bmmw::KMajorLoader<BCOLS>(a.ldb, lane, wave, 0);
+    if constexpr (B_K) return bmmw::KMajorLoader<BCOLS, WAVES>(a.ldb, lane, wave, 0);
     else return lds::MNMajorLoader<256, WAVES>(a.ldb, lane, wave);
   }();
   auto issue_b = [&](int kb) {

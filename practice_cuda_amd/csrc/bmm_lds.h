@@ -58,9 +58,17 @@ PCAMD_DEV void lds_dma16(v4i rs, uint32_t lds, uint32_t voff) {
 // 16-lane group reads 8 k-rows k0..k0+7 (k0 % 8 == 0) at one 8-byte half
 // pair: k & 7 spreads them over 32 banks, and the group served in the same
 // cycle (k-rows 32 further on) lands in the other 32.
-PCAMD_DEV int swz_mn(int k) { return (k & 7) ^ (((k >> 5) & 1) << 3); }
+// 128-byte k-rows (8 chunks): two rows share the 256 bytes, so the eight rows
+// of a group are told apart by bits 1-2 of k and bit 0 (the row's half), and
+// the groups 32 and 64 k-rows apart by chunk bit 2.
+template <int COLS = 256>
+PCAMD_DEV int swz_mn(int k) {
+  if constexpr (COLS == 128) return ((k >> 1) & 3) | ((((k >> 5) ^ (k >> 6)) & 1) << 2);
+  return (k & 7) ^ (((k >> 5) & 1) << 3);
+}
 
-// MN-major tile loader for WAVES waves: 128 k-rows (k0 + k, stride ld) x COLS
+// MN-major tile loader for WAVES waves (128-byte k-rows: an instruction
+// fills eight of them, so one lane offset serves all): 128 k-rows (k0 + k, stride ld) x COLS
 // bytes from col0. Instruction i of wave w fills k-rows kb = w * PER_WAVE +
 // i * R .. + R - 1 (R = 64 / (COLS / 16) rows per instruction); lane l takes
 // k-row kb + l / CHUNKS and LDS slot l % CHUNKS, which holds global chunk
@@ -76,14 +84,14 @@ struct MNMajorLoader {
   static constexpr int R = 64 / CHUNKS;
   static constexpr int PER_WAVE = BK / WAVES;
   static constexpr int INSTS = PER_WAVE / R;
-  static_assert(COLS == 256 && (PER_WAVE == 16 || PER_WAVE == 32),
-                "swizzle assumes 256-byte k-rows, 16 or 32 per wave");
+  static_assert((COLS == 256 && (PER_WAVE == 16 || PER_WAVE == 32)) || (COLS == 128 && PER_WAVE == 32),
+                "swizzle assumes 256-byte k-rows, 16 or 32 per wave, or 128-byte ones, 32 per wave");
   uint32_t voff[2];
   PCAMD_DEV MNMajorLoader(uint32_t ld, int lane, int wave) {
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
       const int k = wave * PER_WAVE + h * R + lane / CHUNKS;
-      voff[h] = (lane / CHUNKS) * ld + (((lane % CHUNKS) ^ swz_mn(k)) << 4);
+      voff[h] = (lane / CHUNKS) * ld + (((lane % CHUNKS) ^ swz_mn<COLS>(k)) << 4);
     }
   }
   PCAMD_DEV void issue(v4i rs, uint8_t* tile, uint32_t col0, uint32_t ld, uint32_t k0, int wave) const {
@@ -121,7 +129,7 @@ PCAMD_DEV v8i frag_mn(const uint8_t* tile, int col16, int lane) {
 #pragma unroll
   for (int q = 0; q < 4; ++q) {
     const int k = 32 * g + 8 * q + (j >> 1);
-    const uint8_t* p = tile + k * COLS + ((c ^ swz_mn(k)) << 4) + half;
+    const uint8_t* p = tile + k * COLS + ((c ^ swz_mn<COLS>(k)) << 4) + half;
     const v2i v = __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_v2i_ptr)(p));
     f[2 * q] = v[0];
     f[2 * q + 1] = v[1];

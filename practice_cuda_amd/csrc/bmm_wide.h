@@ -9,6 +9,9 @@
 // owns 64 x 128 = 4 x 8 tiles of v_mfma_f32_16x16x128_f8f6f4, issued with the
 // operands swapped so a lane holds four consecutive N outputs of one row.
 //
+// Small tiles (SMALL): where 256 x 256 tiles leave CUs idle, 4 waves (2 x 2)
+// of 64 x 64 compute 128 x 128 tiles, two workgroups per CU (small_cost).
+//
 // Half tiles: when the last wave of tiles would fill at most half the CUs
 // (e.g. 896 tiles on 256 CUs), those tiles run as a second launch of
 // 256 x 128 halves, two workgroups per tile, each wave computing 64 x 64
@@ -62,13 +65,19 @@ using lds::lds_dma16;
 using lds::frag_mn;
 typedef float v4f __attribute__((ext_vector_type(4)));
 
-constexpr int NT = 512;
-constexpr int WAVES = NT / 64;
-constexpr int BM = 256, BN = 256, BK = 128;
-constexpr int A_BYTES = BM * BK, B_BYTES = BN * BK;  // 32 KiB each
-constexpr int STAGE = A_BYTES + B_BYTES;
-template <int COLS>
-using MNMajorLoader = lds::MNMajorLoader<COLS, WAVES>;
+// The workgroup of a 256 x 256 tile (8 waves) or, SMALL, of a 128 x 128 one
+// (4 waves, 2 x 2, two workgroups per CU)
+template <bool SMALL>
+struct Geom {
+  static constexpr int NT = SMALL ? 256 : 512;
+  static constexpr int WAVES = NT / 64;
+  static constexpr int WM = SMALL ? 2 : 4;  // waves along M (2 along N)
+  static constexpr int BM = 64 * WM, BN = BM;
+  static constexpr int A_BYTES = BM * 128, B_BYTES = BN * 128;
+  static constexpr int STAGE = A_BYTES + B_BYTES;
+  static constexpr int LDS_BYTES = 2 * STAGE + 2 * (BM + BN) * 4;
+};
+constexpr int BM = Geom<false>::BM, BN = Geom<false>::BN, BK = 128;
 
 // LDS swizzles. gfx950's LDS serves 256 bytes (64 banks) per cycle.
 // K-major tile (128-byte rows): chunk c of row r sits at position c ^ swz_k(r).
@@ -101,7 +110,7 @@ PCAMD_DEV int swz_k(int r) { return (((r >> 1) & 1) * 5) ^ ((r >> 2) & 1); }
 // the instruction's SGPR offset, so no VALU work is issued per load. Rows past
 // the matrix are out of range through the VGPR part alone; for rows inside
 // it, row * ld + k0 + 127 stays below the row's end (k0 < K <= ld).
-template <int ROWS>
+template <int ROWS, int WAVES>
 struct KMajorLoader {
   static constexpr int PER_WAVE = ROWS / WAVES;
   static constexpr int INSTS = PER_WAVE / 8;
@@ -221,21 +230,26 @@ __device__ __attribute__((noinline)) void epilogue_general(void* c, int64_t c_ro
 //     after MFMA (i, 7) has consumed the current one. The last sub-tile's
 //     MFMAs cover the latency of those reads.
 // JN: 16-column sub-tiles per wave - 8 (256 x 256 tiles), 4 (half tiles of
-// a short last wave) or 7 (256 x 224 tiles). CT: C receives the transpose of
+// a short last wave, and SMALL tiles) or 7 (256 x 224 tiles). CT: C receives the transpose of
 // this product (the launcher computes C^T = B^T A^T when 224-column tiles
 // fill the waves better); only plain 16-bit outputs take it.
-template <bool A_K, bool B_K, int FA, int FB, int MODE, int SBK, int JN, bool KT, bool CT = false>
-__global__ __launch_bounds__(NT, 1) void bmm_wide_kernel(FastArgs a) {
+template <bool A_K, bool B_K, int FA, int FB, int MODE, int SBK, int JN, bool KT, bool CT = false, bool SMALL = false>
+__global__ __launch_bounds__(Geom<SMALL>::NT, SMALL ? 2 : 1) void bmm_wide_kernel(FastArgs a) {
+  constexpr int BM = Geom<SMALL>::BM, BN = Geom<SMALL>::BN, WAVES = Geom<SMALL>::WAVES;
+  constexpr int A_BYTES = Geom<SMALL>::A_BYTES, STAGE = Geom<SMALL>::STAGE;
+  static_assert(!SMALL || JN == 4, "64 x 64 wave tiles in a 128 x 128 tile");
+  constexpr bool HALF = JN == 4 && !SMALL;
   static_assert(JN == 8 || JN == 7 || JN == 4, "sub-tiles per wave: 8 (whole tiles), 7 (224-column tiles) or "
                 "4 (half tiles)");
   static_assert(!CT || JN == 7, "the transposed output goes with 224-column tiles");
+  static_assert(JN != 7 || MODE != 0 || SBK != 0, "a wave's 112 columns can lie in two 128-column quant blocks");
   constexpr int TN = JN == 7 ? 224 : BN;  // tile columns
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   float* sa_tile = reinterpret_cast<float*>(smem + 2 * STAGE);  // [2][BM]
   float* sb_tile = sa_tile + 2 * BM;                             // [2][BN]
   const int t = threadIdx.x;
   const int lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
-  const int wm = wave & 3, wn = wave >> 2;  // 4 x 2 waves
+  const int wm = wave % Geom<SMALL>::WM, wn = wave / Geom<SMALL>::WM;  // 4 x 2 waves (SMALL: 2 x 2)
   const int lr = lane & 15, lg = lane >> 4;
 
   // Tile index (tiles ordered as below) and the wave's first column in it.
@@ -244,8 +258,8 @@ __global__ __launch_bounds__(NT, 1) void bmm_wide_kernel(FastArgs a) {
   // workgroups b and b + 8, on the same XCD, so both read its operands
   // through one L2.
   int pid = blockIdx.x;
-  int wcol = wn * 16 * (JN == 4 ? 8 : JN);
-  if constexpr (JN != 4) {
+  int wcol = wn * 16 * (HALF ? 8 : JN);
+  if constexpr (!HALF) {
     if ((a.total_tiles & 7) == 0) pid = (pid & 7) * (a.total_tiles >> 3) + (pid >> 3);
   } else {
     int hsel;
@@ -273,11 +287,13 @@ __global__ __launch_bounds__(NT, 1) void bmm_wide_kernel(FastArgs a) {
 
   const v4i rsa = make_rsrc(a.a + bidx * a.sab, a.a_extent);
   const v4i rsb = make_rsrc(a.b + bidx * a.sbb, a.b_extent);
-  using LA = typename std::conditional<A_K, KMajorLoader<BM>, MNMajorLoader<BM>>::type;
-  using LB = typename std::conditional<B_K, KMajorLoader<BN>, MNMajorLoader<BN>>::type;
+  using KL = KMajorLoader<BM, WAVES>;
+  using ML = lds::MNMajorLoader<BM, WAVES>;
+  using LA = typename std::conditional<A_K, KL, ML>::type;
+  using LB = typename std::conditional<B_K, KL, ML>::type;
   auto make_loader = [&](auto is_k, uint32_t ld, uint32_t origin) {
-    if constexpr (decltype(is_k)::value) return KMajorLoader<BM>(ld, lane, wave, origin);
-    else return MNMajorLoader<BM>(ld, lane, wave);
+    if constexpr (decltype(is_k)::value) return KL(ld, lane, wave, origin);
+    else return ML(ld, lane, wave);
   };
   const LA load_a = make_loader(std::integral_constant<bool, A_K>{}, a.lda, m0);
   const LB load_b = make_loader(std::integral_constant<bool, B_K>{}, a.ldb, n0);
@@ -314,8 +330,8 @@ __global__ __launch_bounds__(NT, 1) void bmm_wide_kernel(FastArgs a) {
   // tile's 256 row scales, waves 4-7 its 256 column scales (the wave index is
   // made scalar so the choice is uniform). Rows / columns past the matrix read
   // the last valid scale; they only feed outputs that are never stored.
-  const bool row_scales = wave < 4;
-  const int slot = t & 255;
+  const bool row_scales = wave < WAVES / 2;
+  const int slot = t & (BM - 1);
   const int s_idx = row_scales ? min(m0 + slot, a.m - 1) : min(n0 + slot, a.n - 1);
   const int64_t s_off = row_scales ? bidx * a.ssab + int64_t(s_idx >> a.qbm_shift) * a.ssa1
                                    : bidx * a.ssbb + int64_t(s_idx >> a.qbn_shift) * a.ssb2;
@@ -323,7 +339,7 @@ __global__ __launch_bounds__(NT, 1) void bmm_wide_kernel(FastArgs a) {
   const float* s_ptr = (row_scales ? a.sa : a.sb) + s_off;
   float* s_tile = (row_scales ? sa_tile : sb_tile) + slot;
   auto load_scale = [&](int ks) -> float { return s_ptr[int64_t(ks) * s_kstride]; };  // qbk == 128
-  auto store_scale = [&](int ks, float v) { s_tile[(ks & 1) * 256] = v; };
+  auto store_scale = [&](int ks, float v) { s_tile[(ks & 1) * BM] = v; };
 
   v4f acc[4][JN];
 #pragma unroll
@@ -727,8 +743,6 @@ __global__ __launch_bounds__(NT, 1) void bmm_wide_kernel(FastArgs a) {
   }
 }
 
-constexpr int LDS_BYTES = 2 * STAGE + 2 * (BM + BN) * 4;
-
 // PCAMD_BMM_T224=0 keeps the 256 x 256 tiling everywhere (read once)
 inline bool transposed_disabled() {
   static const bool off = [] {
@@ -738,18 +752,10 @@ inline bool transposed_disabled() {
   return off;
 }
 
-// PCAMD_BMM_HALVES=0 keeps whole 256 x 256 tiles for small grids (read once)
-inline bool halves_disabled() {
-  static const bool off = [] {
-    const char* e = getenv("PCAMD_BMM_HALVES");
-    return e && e[0] == '0';
-  }();
-  return off;
-}
-
-template <bool A_K, bool B_K, int FA, int FB, int MODE, int SBK, int JN, bool KT, bool CT = false>
+template <bool A_K, bool B_K, int FA, int FB, int MODE, int SBK, int JN, bool KT, bool CT = false, bool SMALL = false>
 int launch_tiles(const FastArgs& a, int grid, hipStream_t st) {
-  auto kern = bmm_wide_kernel<A_K, B_K, FA, FB, MODE, SBK, JN, KT, CT>;
+  constexpr int NT = Geom<SMALL>::NT, LDS_BYTES = Geom<SMALL>::LDS_BYTES;
+  auto kern = bmm_wide_kernel<A_K, B_K, FA, FB, MODE, SBK, JN, KT, CT, SMALL>;
   static std::atomic<uint64_t> configured{0};  // devices whose LDS limit is set
   const int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(kern), LDS_BYTES, st, configured);
   if (rc != 0) return rc;
@@ -757,17 +763,56 @@ int launch_tiles(const FastArgs& a, int grid, hipStream_t st) {
   return check_launch("bmm_wide_kernel");
 }
 
-// One workgroup per tile (one per CU at a time: the LDS stages allow no
-// more). When the last wave of tiles would occupy at most half the CUs, it
-// runs as a second launch of half tiles instead; a grid of at most half as
-// many tiles as CUs runs as half tiles altogether (twice the CUs at work).
+inline int64_t tiles_of(const FastArgs& a, int64_t batch, int rows, int cols) {
+  return batch * ((a.m + rows - 1) / rows) * ((a.n + cols - 1) / cols);
+}
+
+inline FastArgs with_tiles(const FastArgs& a, int64_t batch, int rows, int cols) {
+  FastArgs t = a;
+  t.tiles_m = (a.m + rows - 1) / rows;
+  t.tiles_n = (a.n + cols - 1) / cols;
+  t.tiles_per_batch = t.tiles_m * t.tiles_n;
+  t.total_tiles = static_cast<int32_t>(t.tiles_per_batch * batch);
+  t.tile_base = 0;
+  return t;
+}
+
+// Time of a grid in units of one wave of whole tiles (one per CU): a short
+// last wave runs as half tiles, about 0.85 of a whole one.
+inline double tile_waves(int64_t tiles, int cus) {
+  if (cus <= 0) return 0.0;
+  const int64_t tail = tiles % cus;
+  return double(tiles / cus) + (tail == 0 ? 0.0 : 2 * tail <= cus ? 0.85 : 1.0);
+}
+
+// The same for 128 x 128 tiles, two per CU at a time: half a wave's outputs,
+// at 1.2 (short K) to 1.35 times the cost per output, as each operand byte is
+// loaded for half as many. MI355X, whole tiles (halves where few) -> 128 x 128,
+// us: 2048 x 4096 x 4096 47.3 -> 38.6, 1500 x 4096 x 4096 (channel scales) 38.1
+// -> 28.5, 4 x 578 x 5632 x 1152 30.3 -> 20.9, 80 x 2048 x 640 x 640 187 -> 169,
+// 4096 x 1024 x 512 8.8 -> 7.7; where whole tiles fill their waves they stay
+// ahead: 80 x 2048 x 960 x 640 264 / 277, 8192 x 14336 x 4096 401 / 538, 16 x 512
+// x 1280 x 960 30.1 / 35.2.
+inline double small_cost(int64_t tiles, int k, int cus) {
+  return double((tiles + 2 * cus - 1) / (2 * cus)) * 0.5 * (k <= 2048 ? 1.2 : 1.35);
+}
+
+// One workgroup per 256 x 256 tile (one per CU at a time: the LDS stages allow
+// no more). When the last wave of tiles would occupy at most half the CUs, it
+// runs as a second launch of half tiles instead; where 128 x 128 tiles fill
+// the chip better (small_cost), those run. 256 x 224 tiles for this product
+// (not its transpose) measured slower wherever their wave count was lower: 777
+// x 14336 x 4096 59.9 -> 64 us, 3 x 3228 x 6752 x 384 49.8 -> 60 us.
 template <bool A_K, bool B_K, int FA, int FB, int MODE, int SBK, bool KT>
 int launch_one(const FastArgs& a, hipStream_t st) {
   const int cus = device_cu_count(st);
-  if (cus > 0 && 2 * a.total_tiles <= cus && !halves_disabled()) {
-    FastArgs half = a;
-    half.tile_base = 0;
-    return launch_tiles<A_K, B_K, FA, FB, MODE, SBK, 4, KT>(half, 2 * a.total_tiles, st);
+  const int64_t batch = a.total_tiles / a.tiles_per_batch;
+  if (cus > 0) {
+    const int64_t small = tiles_of(a, batch, Geom<true>::BM, Geom<true>::BN);
+    if (small <= INT32_MAX && small_cost(small, a.k, cus) < tile_waves(a.total_tiles, cus)) {
+      const FastArgs t = with_tiles(a, batch, Geom<true>::BM, Geom<true>::BN);
+      return launch_tiles<A_K, B_K, FA, FB, MODE, SBK, 4, KT, false, true>(t, t.total_tiles, st);
+    }
   }
   const int tail = cus > 0 && a.total_tiles > cus ? a.total_tiles % cus : 0;
   if (tail == 0 || 2 * tail > cus) return launch_tiles<A_K, B_K, FA, FB, MODE, SBK, 8, KT>(a, a.total_tiles, st);
@@ -789,8 +834,7 @@ int launch_one(const FastArgs& a, hipStream_t st) {
 // column tiles, 3.5).
 inline bool transposed_pays(const FastArgs& a, int cus) {
   if (cus <= 0 || a.total_tiles <= cus) return false;
-  const int tail = a.total_tiles % cus;
-  const double now = a.total_tiles / cus + (tail == 0 ? 0.0 : 2 * tail <= cus ? 0.85 : 1.0);
+  const double now = tile_waves(a.total_tiles, cus);
   const int64_t batch = a.total_tiles / a.tiles_per_batch;
   const int64_t t2 = int64_t((a.n + BM - 1) / BM) * ((a.m + 223) / 224) * batch;
   const double alt = double((t2 + cus - 1) / cus) * (224.0 / 256.0);

@@ -18,7 +18,7 @@ pytestmark = pytest.mark.gpu
 E4M3 = torch.float8_e4m3fn
 
 # grids past the K-split kernel's: whole tiles with a short last wave (half
-# tiles), half tiles only; partial tiles in both directions
+# tiles), 128 x 128 tiles; partial tiles in both directions
 SHAPES = [(1, 1000, 2056, 160), (3, 1030, 8200, 256), (2, 512, 8192, 144)]
 
 
