@@ -200,13 +200,14 @@ _PLAIN = (torch.Tensor, nn.Parameter)
 
 def _ops(*tensors):
     """What the layer calls: ``torch.ops.pcamd`` wherever something may look at
-    or stand in for the ops (compilation, a dispatch mode such as a tracer, a
-    counter or selective checkpointing, a function transform, a tensor
-    subclass), else the functions they run, which spares eager steps the
+    or stand in for the ops (compilation, a function or dispatch mode such as a
+    tracer, a counter or selective checkpointing, a function transform, a
+    tensor subclass), else the functions they run, which spares eager steps the
     dispatcher's Python layers (6.5 us of host time per op, six ops per step).
     Either way the same launches on the same stream; only called where autograd
     does not record (inside the autograd function)."""
-    if (torch.compiler.is_compiling() or torch._C._len_torch_dispatch_stack() or torch.is_grad_enabled()
+    if (torch.compiler.is_compiling() or torch._C._len_torch_dispatch_stack()
+            or torch._C._len_torch_function_stack() or torch.is_grad_enabled()
             or torch._C._functorch.peek_interpreter_stack() is not None
             or any(t is not None and type(t) not in _PLAIN for t in tensors)):
         return torch.ops.pcamd

@@ -81,3 +81,26 @@ def test_fake_impls_give_shapes():
         assert q.dtype == torch.float8_e5m2 and s.shape == (1,)
         out = torch.ops.pcamd.tensor_scaled_bmm(a, b, torch.empty(1), None, torch.float32)
         assert out.shape == (2, 64, 96) and out.dtype == torch.float32
+
+
+def test_layer_ops_go_through_the_dispatcher_where_watched():
+    """Function modes and dispatch modes see torch.ops.pcamd; plain eager steps skip it."""
+    from torch.overrides import TorchFunctionMode
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    from practice_cuda_amd.modules import _Direct, _ops
+
+    class Functions(TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    class Dispatch(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    x = torch.zeros(1, 2, 3)
+    with torch.no_grad():
+        assert _ops(x, None) is _Direct
+        for mode in (Functions, Dispatch):
+            with mode():
+                assert _ops(x, None) is torch.ops.pcamd
