@@ -732,12 +732,31 @@ __global__ __launch_bounds__(kAmaxThreads) void tensor_amax_flat_kernel(TensorAr
   }
 }
 
+// PARTS: the quantize pass walks the tensor backwards, so that it meets first
+// what the amax pass read last, and on the XCD whose L2 holds it: consecutive
+// workgroups go to the 8 XCDs in turn, and of a span of 8 amax units workgroup
+// i takes a piece of unit i % 8. The grid is a whole number of spans (the
+// excess finds no chunks and stores nothing). Which workgroup takes a piece
+// does not change a byte. MI355X, rotating inputs, us per call: bf16 [4096,
+// 4096] 20.7 -> 15.5, fp16 [65536, 960] 52.4 -> 47.9, fp16 [18432, 3200] 49.6 ->
+// 45.6, fp32 [7000, 8192] 81.4 -> 80.0, smaller ones unchanged (host-bound).
+constexpr int kTensorCpl = 2;  // chunks per lane
+constexpr int kTensorSpan = 8 * (kAmaxThreads * 8) / (kTensorFlatThreads * kTensorCpl);  // workgroups per 8 amax units
+static_assert(kTensorSpan * kTensorFlatThreads * kTensorCpl == 8 * kAmaxThreads * 8 && kTensorSpan % 8 == 0,
+              "a span is 8 whole amax units");
+
 template <int DT, int FMT, bool NTS, bool UA, bool PARTS>
 __global__ __launch_bounds__(kTensorFlatThreads) void tensor_quant_flat_kernel(TensorArgs a) {
-  constexpr int EB = elem_bytes<DT>(), CPL = 2;
+  constexpr int EB = elem_bytes<DT>(), CPL = kTensorCpl;
   const int64_t chunks = (a.total + 7) / 8;
   const int lane = threadIdx.x & 63;
-  const int64_t u = int64_t(blockIdx.x) * (kTensorFlatThreads / 64) + (threadIdx.x >> 6);
+  int64_t wg = blockIdx.x;
+  if constexpr (PARTS) {
+    const int64_t span = int64_t(gridDim.x) / kTensorSpan - 1 - wg / kTensorSpan;
+    const int in = static_cast<int>(wg % kTensorSpan);
+    wg = (span * 8 + (in & 7)) * (kTensorSpan / 8) + (in >> 3);
+  }
+  const int64_t u = wg * (kTensorFlatThreads / 64) + (threadIdx.x >> 6);
   const int64_t ch0 = u * (CPL * 64) + lane;
   Chunk<DT> cur[CPL];
 #pragma unroll
@@ -1599,7 +1618,8 @@ struct LaunchTensor {
       const int64_t chunks = (a.total + 7) / 8;
       const int agrid = grid_for(chunks, kAmaxThreads * 8, kAmaxGrid);
       const int64_t waves = (chunks + 127) / 128;
-      const int grid = static_cast<int>((waves + kTensorFlatThreads / 64 - 1) / (kTensorFlatThreads / 64));
+      int grid = static_cast<int>((waves + kTensorFlatThreads / 64 - 1) / (kTensorFlatThreads / 64));
+      if (parts) grid = (grid + kTensorSpan - 1) / kTensorSpan * kTensorSpan;
       a.n_parts = agrid;
       if (any) parts ? flat_pass<true, true>(a, agrid, grid, st) : flat_pass<true, false>(a, agrid, grid, st);
       else parts ? flat_pass<false, true>(a, agrid, grid, st) : flat_pass<false, false>(a, agrid, grid, st);

@@ -44,6 +44,28 @@ def test_per_tensor_workspace(dev, shape, dtype):
     assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
 
 
+@pytest.mark.parametrize("total", [262144 - 8, 262144, 262144 + 8, 262144 + 2049, 3 * 262144 - 3, 40 * 262144 + 11])
+def test_per_tensor_workspace_span_edges(dev, total):
+    """The quantize pass takes the tensor in spans of 262144 elements, the last one first: whole
+    spans, a piece more or less, odd ends. Bytes and scales as without a workspace, nothing behind the end."""
+    x = _x((1, 1, total), torch.bfloat16, dev)
+    L, st = _lib.lib(), _lib.stream_of(x)
+    got = []
+    for ws in (False, True):
+        buf = torch.full((total + 64,), 0x55, dtype=torch.uint8, device=dev)
+        y = buf[:total].view(torch.float8_e4m3fn).view(1, 1, total)
+        s = torch.full((4 + 256,), float("nan"), device=dev)
+        args = (*_head(x, y), s.data_ptr(), s.data_ptr() + 4, 448.0, 1e-12, _lib.F32)
+        if ws:
+            rc = L.pcamd_quant_tensor_ws(*args, 0, s.data_ptr() + 16, 1024, st)
+        else:
+            rc = L.pcamd_quant_tensor(*args, st)
+        _lib.check(rc, "per-tensor")
+        torch.cuda.synchronize()
+        got.append((buf, s[:2].view(torch.int32)))
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
+
+
 @pytest.mark.parametrize("shape", [(1, 257, 8), (1, 300, 130), (2, 1281, 264), (1, 4300, 1024), (3, 700, 1031)])
 def test_per_column_workspace(dev, shape):
     """Parts of one slab and of several, a ragged last part, batches, odd rows."""
