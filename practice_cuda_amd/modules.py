@@ -196,20 +196,37 @@ class _Direct:
 
 
 _PLAIN = (torch.Tensor, nn.Parameter)
+_OPS = (block_scaled_bmm, tensor_scaled_bmm, quant_block, quant_block_dual, quant_tensor)
+_OWN_KERNELS = tuple(dict(op._backend_fns) for op in _OPS)
+
+
+def _plain(t: Optional[torch.Tensor]) -> bool:
+    """Whether the dispatcher would hand t to the ops' functions as it is: no
+    subclass, no meta tensor (the fake implementations answer for those), no
+    lazy negation or zero that it materializes first."""
+    return t is None or (type(t) in _PLAIN and not (t.is_meta or t.is_neg() or t._is_zerotensor()))
+
+
+def _replaced() -> bool:
+    """Whether a kernel or an autocast rule was registered on one of the ops."""
+    return any(op._backend_fns != own or op._autocast_cuda_dtype is not None
+               or torch._C._dispatch_has_kernel_for_dispatch_key(op._qualname, "CUDA")
+               for op, own in zip(_OPS, _OWN_KERNELS))
 
 
 def _ops(*tensors):
-    """What the layer calls: ``torch.ops.pcamd`` wherever something may look at
-    or stand in for the ops (compilation, a function or dispatch mode such as a
-    tracer, a counter or selective checkpointing, a function transform, a
-    tensor subclass), else the functions they run, which spares eager steps the
-    dispatcher's Python layers (6.5 us of host time per op, six ops per step).
-    Either way the same launches on the same stream; only called where autograd
-    does not record (inside the autograd function)."""
-    if (torch.compiler.is_compiling() or torch._C._len_torch_dispatch_stack()
-            or torch._C._len_torch_function_stack() or torch.is_grad_enabled()
-            or torch._C._functorch.peek_interpreter_stack() is not None
-            or any(t is not None and type(t) not in _PLAIN for t in tensors)):
+    """What the layer calls: ``torch.ops.pcamd`` wherever something looks at or
+    stands in for the ops (compilation or tracing, a function or dispatch mode
+    such as a counter or selective checkpointing, a function transform, a
+    profiler, a kernel registered on an op, a tensor that is not plain), else
+    the functions they run, which spares eager steps the dispatcher's Python
+    layers (6.5 us of host time per op, six ops per step). Either way the same
+    launches on the same stream; only called where autograd does not record
+    (inside the autograd function)."""
+    if (torch.compiler.is_compiling() or torch._C._get_tracing_state() is not None
+            or torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack()
+            or torch.is_grad_enabled() or torch._C._functorch.peek_interpreter_stack() is not None
+            or torch.autograd._profiler_enabled() or not all(map(_plain, tensors)) or _replaced()):
         return torch.ops.pcamd
     return _Direct
 
@@ -260,7 +277,7 @@ class _Float8BlockBMMLinearFunction(torch.autograd.Function):
     def forward(ctx, input: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor],
                 config: Float8BlockBMMLinearConfig) -> torch.Tensor:
         f8, eps, blk = config.fp8_dtype, config.eps, config.block
-        ops = _ops(input, weight)
+        ops = _ops(input, weight, bias)
         ctx.config = config
         ctx.has_bias = bias is not None
         bias_k = None if bias is None else bias.to(input.dtype)

@@ -104,3 +104,74 @@ def test_layer_ops_go_through_the_dispatcher_where_watched():
         for mode in (Functions, Dispatch):
             with mode():
                 assert _ops(x, None) is torch.ops.pcamd
+
+
+@pytest.mark.parametrize("granularity", ["block", "tensor"])
+def test_layer_on_meta_tensors(granularity):
+    """Shapes, dtypes and gradients without a device: the ops' fake implementations answer."""
+    layer = Float8BMMLinear(2, 256, 384, config=Float8BlockBMMLinearConfig(granularity=granularity), device="meta",
+                            dtype=torch.bfloat16)
+    x = torch.empty(2, 40, 256, device="meta", dtype=torch.bfloat16, requires_grad=True)
+    y = layer(x)
+    assert y.is_meta and y.shape == (2, 40, 384) and y.dtype == torch.bfloat16
+    grads = torch.autograd.grad(y, [x, layer.weight, layer.bias], torch.empty_like(y))
+    assert [g.shape for g in grads] == [x.shape, layer.weight.shape, layer.bias.shape]
+
+
+def test_layer_ops_go_through_the_dispatcher_for_tensors_it_prepares():
+    """A subclass, a lazily negated view and an unmaterialized zero: the dispatcher hands the op another tensor."""
+    from practice_cuda_amd.modules import _Direct, _ops
+
+    class Sub(torch.Tensor):
+        pass
+
+    x = torch.zeros(1, 2, 3)
+    negated = torch.zeros(1, 2, 3, dtype=torch.complex64).conj().imag
+    assert negated.is_neg()
+    with torch.no_grad():
+        assert _ops(x, None) is _Direct
+        for t in (x.as_subclass(Sub), x.to("meta"), negated, torch._efficientzerotensor(1, 2, 3)):
+            assert _ops(x, x, t) is torch.ops.pcamd
+
+
+def test_layer_passes_its_bias_to_the_dispatch_check(monkeypatch):
+    """The bias is an operand of the product as well."""
+    from practice_cuda_amd import modules
+
+    seen = []
+    monkeypatch.setattr(modules, "_ops", lambda *tensors: seen.append(tensors) or torch.ops.pcamd)
+    layer = Float8BMMLinear(1, 128, 128, device="meta", dtype=torch.bfloat16)
+    layer(torch.empty(1, 4, 128, device="meta", dtype=torch.bfloat16))
+    assert any(t is layer.bias or t.shape == layer.bias.shape for t in seen[0])
+
+
+def test_layer_ops_go_through_the_dispatcher_under_a_profiler_and_tracing():
+    from practice_cuda_amd.modules import _Direct, _ops
+
+    x = torch.zeros(1, 2, 3)
+    with torch.no_grad():
+        with torch.profiler.profile():
+            assert _ops(x) is torch.ops.pcamd
+        traced = []
+        torch.jit.trace(lambda t: traced.append(_ops(t)) or t * 2, (x,), check_trace=False)
+        assert traced == [torch.ops.pcamd]
+        assert _ops(x) is _Direct
+
+
+def test_layer_ops_go_through_the_dispatcher_where_a_kernel_was_registered():
+    """Registrations last for the process, so each runs in one of its own."""
+    import os
+    import subprocess
+    import sys
+
+    prologue = "import torch; from practice_cuda_amd import modules as M; x = torch.zeros(1)\n"
+    check = ("with torch.no_grad():\n    assert M._ops(x) is M._Direct\n    {}\n"
+             "    assert M._ops(x) is torch.ops.pcamd\n")
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    for register in ("M.quant_block.register_kernel('cuda')(lambda *a: None)",
+                     "torch.library.register_kernel('pcamd::quant_tensor', 'cuda', lambda *a: None)",
+                     "lib = torch.library.Library('pcamd', 'IMPL'); lib.impl('block_scaled_bmm', lambda *a: None, 'CUDA')",
+                     "M.tensor_scaled_bmm.register_autocast('cuda', torch.bfloat16)"):
+        run = subprocess.run([sys.executable, "-c", prologue + check.format(register)], cwd=root, capture_output=True,
+                             text=True, timeout=300)
+        assert run.returncode == 0, register + "\n" + run.stderr
