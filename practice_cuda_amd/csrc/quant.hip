@@ -141,6 +141,22 @@ PCAMD_DEV void store8_n(uint8_t* p, uint2 v, int64_t nv) {
   }
 }
 
+// max |x| over a chunk's elements. SKIP: NaN elements do not count, whatever
+// the type, as in the element-wise kernels (chunk_amax orders bf16 by its bits,
+// so a NaN there is the largest value).
+template <int DT, bool SKIP>
+PCAMD_DEV float chunk_amax_n(const Chunk<DT>& c) {
+  if constexpr (!SKIP) {
+    return chunk_amax<DT>(c);
+  } else {
+    float v[8], amax = 0.0f;
+    unpack_chunk<DT>(c, v);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) amax = fmaxf(amax, fabsf(v[i]));
+    return amax;
+  }
+}
+
 // 1 x (8 * LPG) groups along a row. A unit is CPL * 64 consecutive chunks of
 // one row; each wave quantizes one unit (kGroupThreads / 64 units per
 // workgroup). FLAT: input, output and scales are contiguous and the row
@@ -196,7 +212,7 @@ __global__ __launch_bounds__(kGroupThreads) void quant_groups_kernel(RowArgs a) 
 #pragma unroll
   for (int c = 0; c < CPL; ++c) {
     const int ch = chunk0 + c * 64;
-    const float amax = group_max<LPG>(chunk_amax<DT>(cur[c]));
+    const float amax = group_max<LPG>(chunk_amax_n<DT, UA>(cur[c]));
     const Scales s = block_scales(amax, a.fp8_max, a.eps);
     if (ch < a.chunks) {
       if ((lane & (LPG - 1)) == 0) srow[int64_t(ch / LPG) * a.ssn] = s.ds;
@@ -225,7 +241,7 @@ __global__ __launch_bounds__(kThreads) void quant_waverow_kernel(RowArgs a) {
   }
   float amax = 0.0f;
 #pragma unroll
-  for (int c = 0; c < MAXC; ++c) amax = fmaxf(amax, chunk_amax<DT>(raw[c]));
+  for (int c = 0; c < MAXC; ++c) amax = fmaxf(amax, chunk_amax_n<DT, UA>(raw[c]));
   amax = group_max<64>(amax);
   const Scales s = channel_scales(amax, a.fp8_max, a.eps);
   if (lane == 0) a.scale[int64_t(b) * a.ssb + int64_t(mi) * a.ssm] = s.ds;
@@ -268,7 +284,7 @@ __global__ __launch_bounds__(1024) void quant_rowblock_kernel(RowArgs a) {
   }
   float amax = 0.0f;
 #pragma unroll
-  for (int c = 0; c < CPT; ++c) amax = fmaxf(amax, chunk_amax<DT>(cur[c]));
+  for (int c = 0; c < CPT; ++c) amax = fmaxf(amax, chunk_amax_n<DT, UA>(cur[c]));
   amax = group_max<64>(amax);
   if ((t & 63) == 0) red[t >> 6] = amax;
   __syncthreads();
@@ -331,7 +347,7 @@ __global__ __launch_bounds__(kThreads) void quant_tile_kernel(TileArgs a) {
     }
     float amax = 0.0f;
 #pragma unroll
-    for (int p = 0; p < CPT; ++p) amax = fmaxf(amax, chunk_amax<DT>(cur[p]));
+    for (int p = 0; p < CPT; ++p) amax = fmaxf(amax, chunk_amax_n<DT, UA>(cur[p]));
     amax = group_max<64>(amax);
     if ((t & 63) == 0) rd[t >> 6] = amax;
     __syncthreads();
@@ -699,7 +715,8 @@ constexpr int kAmaxGrid = 256;
 // MI355X, fp16 [65536, 960], with the scale's cast to fp16 in the same launch and
 // the amax pass reading with ordinary loads (the quantize pass finds part of the
 // tensor in cache): 56.0 -> 52.3 us per call.
-template <int DT, bool UA, bool PARTS>
+// SKIP: runs that the element-wise kernel would take by their rows (chunk_amax_n).
+template <int DT, bool UA, bool PARTS, bool SKIP>
 __global__ __launch_bounds__(kAmaxThreads) void tensor_amax_flat_kernel(TensorArgs a) {
   constexpr int EB = elem_bytes<DT>(), CPT = 8, W = kAmaxThreads / 64;
   __shared__ float red[W];
@@ -719,7 +736,7 @@ __global__ __launch_bounds__(kAmaxThreads) void tensor_amax_flat_kernel(TensorAr
       }
     }
 #pragma unroll
-    for (int p = 0; p < CPT; ++p) amax = fmaxf(amax, chunk_amax<DT>(c[p]));
+    for (int p = 0; p < CPT; ++p) amax = fmaxf(amax, chunk_amax_n<DT, SKIP>(c[p]));
   }
   amax = group_max<64>(amax);
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = amax;
@@ -1605,13 +1622,15 @@ struct LaunchGeneric {
 template <int DT, int FMT>
 struct LaunchTensor {
   template <bool UA, bool PARTS>
-  static void flat_pass(const TensorArgs& a, int agrid, int grid, hipStream_t st) {
-    tensor_amax_flat_kernel<DT, UA, PARTS><<<agrid, kAmaxThreads, 0, st>>>(a);
+  static void flat_pass(const TensorArgs& a, bool rows, int agrid, int grid, hipStream_t st) {
+    if (UA || !rows) tensor_amax_flat_kernel<DT, UA, PARTS, true><<<agrid, kAmaxThreads, 0, st>>>(a);
+    else tensor_amax_flat_kernel<DT, UA, PARTS, UA><<<agrid, kAmaxThreads, 0, st>>>(a);
     if (!UA && nt_stores()) tensor_quant_flat_kernel<DT, FMT, !UA, UA, PARTS><<<grid, kTensorFlatThreads, 0, st>>>(a);
     else tensor_quant_flat_kernel<DT, FMT, false, UA, PARTS><<<grid, kTensorFlatThreads, 0, st>>>(a);
   }
-  // flat: one contiguous run of elements; any: not of whole aligned chunks
-  static int run(TensorArgs a, bool flat, bool any, hipStream_t st) {
+  // flat: one contiguous run of elements; any: not of whole aligned chunks;
+  // rows: its rows are of whole aligned chunks too
+  static int run(TensorArgs a, bool flat, bool any, bool rows, hipStream_t st) {
     const bool parts = flat && a.total > 0 && a.parts != nullptr;
     if (!parts) fill_zero_u32_kernel<<<1, 1, 0, st>>>(reinterpret_cast<uint32_t*>(a.scale));
     if (a.total > 0 && flat) {
@@ -1621,8 +1640,8 @@ struct LaunchTensor {
       int grid = static_cast<int>((waves + kTensorFlatThreads / 64 - 1) / (kTensorFlatThreads / 64));
       if (parts) grid = (grid + kTensorSpan - 1) / kTensorSpan * kTensorSpan;
       a.n_parts = agrid;
-      if (any) parts ? flat_pass<true, true>(a, agrid, grid, st) : flat_pass<true, false>(a, agrid, grid, st);
-      else parts ? flat_pass<false, true>(a, agrid, grid, st) : flat_pass<false, false>(a, agrid, grid, st);
+      if (any) parts ? flat_pass<true, true>(a, rows, agrid, grid, st) : flat_pass<true, false>(a, rows, agrid, grid, st);
+      else parts ? flat_pass<false, true>(a, rows, agrid, grid, st) : flat_pass<false, false>(a, rows, agrid, grid, st);
     } else if (a.total > 0) {
       const int grid = grid_for(a.total, kThreads, 4096);
       tensor_amax_kernel<DT><<<grid, kThreads, 0, st>>>(a);
@@ -1981,7 +2000,7 @@ static int quant_tensor(const void* x, int x_dtype, int64_t batch, int64_t m, in
                     (batch == 1 || (sxb == m * n && syb == m * n)) && (a.total / 8 + 128) / 128 < (1LL << 31);
   // (a run of whole chunks may be made of rows that are not)
   const bool whole = a.total % 8 == 0 && aligned(x, 16) && aligned(y, 8);
-  return dispatch_dt_fmt<LaunchTensor>(x_dtype, y_dtype, a, flat, !whole, static_cast<hipStream_t>(stream));
+  return dispatch_dt_fmt<LaunchTensor>(x_dtype, y_dtype, a, flat, !whole, fast, static_cast<hipStream_t>(stream));
 }
 
 extern "C" int pcamd_quant_tensor(const void* x, int x_dtype, int64_t batch, int64_t m, int64_t n, int64_t sxb,

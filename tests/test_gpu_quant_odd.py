@@ -75,3 +75,28 @@ def test_odd_e5m2_reduced_range(dev):
     x = torch.randn(33, 1031, generator=torch.Generator().manual_seed(4))
     q, s = fp8_quant(x.to(dev), fp8_range=100.0)
     _same(q, s, *O.quant_tensor(x, scale_dt="input", fp8_max=100.0)[:2], "legacy fp8_range")
+
+
+@pytest.mark.parametrize("dtype", ["bf16", "f16", "f32"])
+def test_odd_rows_skip_nan_in_the_maxima(dev, dtype):
+    """A NaN does not count in the maximum of what it is quantized with, and no
+    other element's byte depends on it: every scale and byte but its own are
+    those of the tensor with 0 in its place. (128 consecutive NaN: whole chunks
+    and a whole group of them; [8, 1031] is also one run of whole chunks.)"""
+    x = torch.randn(8, 1031, generator=torch.Generator().manual_seed(5)).to(DT[dtype])
+    nan = torch.zeros(x.shape, dtype=torch.bool)
+    nan[0, 3] = nan[1, 256:384] = nan[2, 1030] = nan[3, 8:16] = True
+    clean, dirty = x.masked_fill(nan, 0.0).to(dev), x.masked_fill(nan, float("nan")).to(dev)
+    nan = nan.to(dev)
+    cases = {f"block {bm}x{bn}": lambda t, bm=bm, bn=bn: hip_per_block_quant(t, block_m=bm, block_n=bn)
+             for bm, bn in ((1, 8), (1, 128), (1, 512), (128, 128), (16, 64))}
+    cases.update({f"channel {a}": lambda t, a=a: hip_per_channel_quant(t, channel_axis=a) for a in (-2, -1)})
+    cases["tensor"] = hip_per_tensor_quant
+    for name, fn in cases.items():
+        print(f"odd rows NaN {name} {dtype}", flush=True)
+        want, got = fn(clean), fn(dirty)
+        assert torch.equal(want.dequant_scale, got.dequant_scale), name
+        assert torch.equal(want.tensor.view(torch.uint8)[~nan], got.tensor.view(torch.uint8)[~nan]), name
+    want, got = fp8_quant(clean), fp8_quant(dirty)
+    assert torch.equal(want[1], got[1])
+    assert torch.equal(want[0].view(torch.uint8)[~nan], got[0].view(torch.uint8)[~nan])
