@@ -197,21 +197,16 @@ class _Direct:
 
 _PLAIN = (torch.Tensor, nn.Parameter)
 _OPS = (block_scaled_bmm, tensor_scaled_bmm, quant_block, quant_block_dual, quant_tensor)
-_OWN_KERNELS = tuple(dict(op._backend_fns) for op in _OPS)
+_OWN_KERNELS = tuple(op._backend_fns[None] for op in _OPS)
+# torch.library's record of what was registered on ops from Python
+_REGISTERED = torch.library._impls
+_OVERRIDES = frozenset(f"{op._qualname.replace('::', '/')}/{key}" for op in _OPS
+                       for key in ("CUDA", "AutogradCUDA", "AutocastCUDA"))
 
 
-def _plain(t: Optional[torch.Tensor]) -> bool:
-    """Whether the dispatcher would hand t to the ops' functions as it is: no
-    subclass, no meta tensor (the fake implementations answer for those), no
-    lazy negation or zero that it materializes first."""
-    return t is None or (type(t) in _PLAIN and not (t.is_meta or t.is_neg() or t._is_zerotensor()))
-
-
-def _replaced() -> bool:
-    """Whether a kernel or an autocast rule was registered on one of the ops."""
-    return any(op._backend_fns != own or op._autocast_cuda_dtype is not None
-               or torch._C._dispatch_has_kernel_for_dispatch_key(op._qualname, "CUDA")
-               for op, own in zip(_OPS, _OWN_KERNELS))
+_tracing, _profiling = torch._C._get_tracing_state, torch.autograd._profiler_enabled
+_dispatch_modes, _function_modes = torch._C._len_torch_dispatch_stack, torch._C._len_torch_function_stack
+_transforms, _recording = torch._C._functorch.peek_interpreter_stack, torch.is_grad_enabled
 
 
 def _ops(*tensors):
@@ -223,11 +218,16 @@ def _ops(*tensors):
     layers (6.5 us of host time per op, six ops per step). Either way the same
     launches on the same stream; only called where autograd does not record
     (inside the autograd function)."""
-    if (torch.compiler.is_compiling() or torch._C._get_tracing_state() is not None
-            or torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack()
-            or torch.is_grad_enabled() or torch._C._functorch.peek_interpreter_stack() is not None
-            or torch.autograd._profiler_enabled() or not all(map(_plain, tensors)) or _replaced()):
+    if (torch.compiler.is_compiling() or _tracing() is not None or _dispatch_modes() or _function_modes()
+            or _recording() or _transforms() is not None or _profiling()
+            or not _OVERRIDES.isdisjoint(_REGISTERED)
+            or tuple([op._backend_fns[None] for op in _OPS]) != _OWN_KERNELS):
         return torch.ops.pcamd
+    for t in tensors:
+        # the dispatcher hands the ops' functions another tensor: it calls the fake implementations for
+        # meta tensors and materializes lazy negations and zeros first
+        if t is not None and (type(t) not in _PLAIN or t.is_meta or t.is_neg() or t._is_zerotensor()):
+            return torch.ops.pcamd
     return _Direct
 
 
