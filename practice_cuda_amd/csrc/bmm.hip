@@ -528,6 +528,11 @@ static int bmm_scaled(const void* a, int a_fmt, const void* b, int b_fmt, int64_
     const char* e = getenv("PCAMD_BMM_STREAM");
     return e && e[0] == '0';
   }();
+  // past 2^32 threads in a grid dimension a launch reports nothing and runs the remainder only
+  auto launch_general = [&]() -> int {
+    if (args.total_tiles > UINT32_MAX / bmm::NT) return set_error(PCAMD_ERR_UNSUPPORTED, "too many output tiles");
+    return bmm::launch_formats(args, a_fmt, b_fmt, a_k, b_k, mode, st);
+  };
   {
     // K not a multiple of 128: the wide kernel masks its last K step (two
     // steps or more, K a multiple of 4); the other fast kernels need whole steps
@@ -576,14 +581,15 @@ static int bmm_scaled(const void* a, int a_fmt, const void* b, int b_fmt, int64_
           bmm_stream_ok(f, a_k, b_k, fmode, batch, args.qbm, args.qbn, ssa1, ssb2))
         return bmm_stream_launch(f, a_fmt, batch, st);
       // products of several K steps on a short grid, and unaligned operands
-      if (bmm_split_ok(f, a_fmt, b_fmt, a_k, b_k, fmode, batch) &&
+      if (bmm_split_ok(f, a_fmt, b_fmt, a_k, b_k, fmode, batch, st) &&
           (!fast || (wide && bmm_split_pays(f, batch, st))))
         return bmm_split_launch(f, a_k, b_k, fmode, batch, st);
+      if (tm * tn * batch > UINT32_MAX / 512) return launch_general();
       if (fast && wide) return bmm_wide_launch(f, a_fmt, b_fmt, a_k, b_k, fmode, st);
       if (fast && same_fmt) return bmm_fast_launch(f, a_fmt, a_k, b_k, fmode, sb_col, qb1, st);
     }
   }
-  return bmm::launch_formats(args, a_fmt, b_fmt, a_k, b_k, mode, st);
+  return launch_general();
 }
 
 extern "C" int pcamd_bmm_scaled(const void* a, const void* b, int ab_dtype, int64_t batch, int64_t m,

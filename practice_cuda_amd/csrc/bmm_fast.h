@@ -75,7 +75,8 @@ int bmm_wide_tile();
 // e4m3fn operands, quant-K 128 in block mode, rows of at least 16 bytes;
 // bmm_split_pays whether it is ahead of the tiled kernels on operands that
 // those take too. It uses a's strides, extents and sizes, not its tile counts.
-bool bmm_split_ok(const FastArgs& a, int a_fmt, int b_fmt, bool a_k, bool b_k, int mode, int64_t batch);
+bool bmm_split_ok(const FastArgs& a, int a_fmt, int b_fmt, bool a_k, bool b_k, int mode, int64_t batch,
+                  hipStream_t st);
 bool bmm_split_pays(const FastArgs& a, int64_t batch, hipStream_t st);
 int bmm_split_launch(const FastArgs& a, bool a_k, bool b_k, int mode, int64_t batch, hipStream_t st);
 

@@ -7,6 +7,9 @@ namespace bmmp {
 
 // 16 x 16 sub-tiles (MI x NJ) and waves of a workgroup
 enum Shape { k1x2w8, k1x4w4, k1x4w8, k2x2w8, k2x4w4, k2x4w8, k4x4w4, k4x4w8 };
+struct Tile { int rows, cols, threads; };
+constexpr Tile kTiles[] = {{16, 32, 512}, {16, 64, 256}, {16, 64, 512}, {32, 32, 512},
+                           {32, 64, 256}, {32, 64, 512}, {64, 64, 256}, {64, 64, 512}};
 
 inline int64_t tiles(const FastArgs& a, int64_t batch, int rows, int cols) {
   return batch * ((a.m + rows - 1) / rows) * ((a.n + cols - 1) / cols);
@@ -69,11 +72,16 @@ int launch_mode(const FastArgs& a, int mode, int64_t batch, hipStream_t st) {
 
 }  // namespace bmmp
 
-bool bmm_split_ok(const FastArgs& a, int a_fmt, int b_fmt, bool a_k, bool b_k, int mode, int64_t batch) {
+bool bmm_split_ok(const FastArgs& a, int a_fmt, int b_fmt, bool a_k, bool b_k, int mode, int64_t batch,
+                  hipStream_t st) {
   if (a_fmt != kE4M3 || b_fmt != kE4M3) return false;
   // a 16-byte piece must fit in the rows that are walked
   if (((a_k || b_k) && a.k < 16) || (!a_k && a.m < 16) || (!b_k && a.n < 16)) return false;
-  if (batch * ((a.m + 15) / 16) * int64_t((a.n + 31) / 32) >= INT32_MAX) return false;
+  // sizes rounded up to a tile, and a launch's threads, fit 32 bits (many small batches: the
+  // general kernel's 128 x 128 tiles and 256 threads reach further)
+  if (a.m > INT32_MAX - 64 || a.n > INT32_MAX - 64) return false;
+  const bmmp::Tile t = bmmp::kTiles[bmmp::pick(a, batch, device_cu_count(st), mode == 0)];
+  if (bmmp::tiles(a, batch, t.rows, t.cols) > UINT32_MAX / t.threads) return false;
   if (mode == 0) {
     if (a.qbk != 128 || a.qbm_shift < 0 || a.qbn_shift < 0) return false;
     const int64_t ra = int64_t((a.m - 1) >> a.qbm_shift) * a.ssa1, rb = int64_t((a.n - 1) >> a.qbn_shift) * a.ssb2;

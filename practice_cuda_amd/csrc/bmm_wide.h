@@ -809,7 +809,7 @@ int launch_one(const FastArgs& a, hipStream_t st) {
   const int64_t batch = a.total_tiles / a.tiles_per_batch;
   if (cus > 0) {
     const int64_t small = tiles_of(a, batch, Geom<true>::BM, Geom<true>::BN);
-    if (small <= INT32_MAX && small_cost(small, a.k, cus) < tile_waves(a.total_tiles, cus)) {
+    if (small <= UINT32_MAX / Geom<true>::NT && small_cost(small, a.k, cus) < tile_waves(a.total_tiles, cus)) {
       const FastArgs t = with_tiles(a, batch, Geom<true>::BM, Geom<true>::BN);
       return launch_tiles<A_K, B_K, FA, FB, MODE, SBK, 4, KT, false, true>(t, t.total_tiles, st);
     }

@@ -1294,6 +1294,10 @@ __global__ __launch_bounds__(NT) void quant_dual_kernel(DualArgs a) {
 // ===========================================================================
 // host dispatch helpers
 // ===========================================================================
+// A grid dimension holds fewer than 2^32 threads: past that a launch reports
+// nothing and runs the remainder only.
+inline bool launchable(int64_t blocks, int64_t threads) { return blocks <= UINT32_MAX / threads; }
+
 inline int grid_for(int64_t units, int64_t per_block = 1, int64_t cap = 1 << 20) {
   int64_t g = (units + per_block - 1) / per_block;
   return static_cast<int>(std::max<int64_t>(1, std::min<int64_t>(g, cap)));
@@ -1405,6 +1409,12 @@ struct LaunchGroups {
   }
 };
 
+// threads of a row: a wave, or a workgroup with two or (always in the UA
+// kernels) four chunks per lane
+inline int row_threads(int64_t chunks, int cpt = 4) {
+  return chunks < 256 ? 64 : static_cast<int>(((chunks + cpt - 1) / cpt + 63) / 64 * 64);
+}
+
 template <int DT, int FMT>
 struct LaunchRowBlock {
   template <int CPT, bool NTS>
@@ -1437,8 +1447,8 @@ struct LaunchRowBlock {
     // on, equal at 4096 and 8192, two per lane 1 % faster at 2048 (7168: 256
     // threads, 63.4 -> 61.5 us on the config-2 tensor).
     if (a.chunks < 256) return wave<4, NTS>(a, st);
-    if (a.chunks <= 512) return go<2, NTS>(a, ((a.chunks + 1) / 2 + 63) / 64 * 64, st);
-    return go<4, NTS>(a, ((a.chunks + 3) / 4 + 63) / 64 * 64, st);  // <= 512 threads: chunks <= 2048
+    if (a.chunks <= 512) return go<2, NTS>(a, row_threads(a.chunks, 2), st);
+    return go<4, NTS>(a, row_threads(a.chunks), st);  // <= 512 threads: chunks <= 2048
   }
   static int run(const RowArgs& a, hipStream_t st) {
     if (a.n > 0) {  // rows of any length and alignment
@@ -1446,8 +1456,7 @@ struct LaunchRowBlock {
         quant_waverow_kernel<DT, FMT, 4, false, true><<<static_cast<int>((int64_t(a.units) + 3) / 4), kThreads, 0, st>>>(a);
         return check_launch("quant_waverow_kernel");
       }
-      const int threads = ((a.chunks + 3) / 4 + 63) / 64 * 64;
-      quant_rowblock_kernel<DT, FMT, 4, false, false, true, true><<<a.units, threads, 0, st>>>(a);
+      quant_rowblock_kernel<DT, FMT, 4, false, false, true, true><<<a.units, row_threads(a.chunks), 0, st>>>(a);
       return check_launch("quant_rowblock_kernel");
     }
     return nt_stores() ? pick<true>(a, st) : pick<false>(a, st);
@@ -1738,7 +1747,7 @@ extern "C" int pcamd_quant_block(const void* x, int x_dtype, int64_t batch, int6
     a.cpl = cpl;
     a.fp8_max = fp8_max; a.eps = eps;
     const int64_t units = flat ? (a.total + 127) / 128 : int64_t(batch) * m * a.segs;
-    if (units < UINT32_MAX) return dispatch_dt_fmt<LaunchGroups>(x_dtype, y_dtype, a, lpg, cpl, st);
+    if (launchable((units + 3) / 4, kGroupThreads)) return dispatch_dt_fmt<LaunchGroups>(x_dtype, y_dtype, a, lpg, cpl, st);
   }
   const int64_t lpr = block_n / 8;
   if (rows && block_n >= 32 && lpr <= 64 && (block_m * lpr) % kThreads == 0 &&
@@ -1907,7 +1916,8 @@ static int quant_channel(const void* x, int x_dtype, int64_t batch, int64_t m, i
     a.fp8_max = fp8_max; a.eps = eps;
     return dispatch_dt_fmt<LaunchGeneric>(x_dtype, y_dtype, a, 2, st);
   }
-  if (channel_axis == -2 && rows && (n + 7) / 8 <= 8LL * kThreads && batch * m < INT32_MAX && m < UINT32_MAX) {
+  if (channel_axis == -2 && rows && (n + 7) / 8 <= 8LL * kThreads && batch * m < INT32_MAX && m < UINT32_MAX &&
+      launchable((batch * m + 3) / 4 * 4, row_threads((n + 7) / 8, fast && n <= 4096 ? 2 : 4))) {
     RowArgs a{};
     a.x = static_cast<const char*>(x); a.y = static_cast<uint8_t*>(y); a.scale = scale;
     a.m = static_cast<uint32_t>(m); a.sxb = sxb; a.sxm = sxm; a.syb = syb; a.sym = sym;
@@ -1931,8 +1941,8 @@ static int quant_channel(const void* x, int x_dtype, int64_t batch, int64_t m, i
     // Tall tensors: 128-row slabs in parallel (column maxima by atomic max in
     // the scale slots, then a quantize pass). Up to 256 rows one workgroup
     // per strip reads its rows twice.
-    if ((m > 256 || !fast) && a.strips <= INT32_MAX && (m + 127) / 128 <= 65535 && batch <= 65535 &&
-        (batch * n + kThreads - 1) / kThreads <= INT32_MAX) {
+    if ((m > 256 || !fast) && launchable(a.strips, kThreads) && (m + 127) / 128 <= 65535 && batch <= 65535 &&
+        launchable((batch * n + kThreads - 1) / kThreads, kThreads)) {
       if (workspace) {
         const ColParts p = col_parts(batch, m, n);
         if (!aligned(workspace, 4) || workspace_bytes < batch * p.parts * n * 4)
@@ -1997,7 +2007,8 @@ static int quant_tensor(const void* x, int x_dtype, int64_t batch, int64_t m, in
   // one contiguous run of elements in and out, of whole aligned chunks or not
   const bool fast = row_fast_ok(x, x_dtype, y, n, sxb, sxm, sxn, syb, sym, syn);
   const bool flat = (fast || row_any_ok(n, sxn, syn)) && (m == 1 || (sxm == n && sym == n)) &&
-                    (batch == 1 || (sxb == m * n && syb == m * n)) && (a.total / 8 + 128) / 128 < (1LL << 31);
+                    (batch == 1 || (sxb == m * n && syb == m * n)) &&
+                    launchable(a.total / (8 * 2 * kTensorFlatThreads) + kTensorSpan + 1, kTensorFlatThreads);
   // (a run of whole chunks may be made of rows that are not)
   const bool whole = a.total % 8 == 0 && aligned(x, 16) && aligned(y, 8);
   return dispatch_dt_fmt<LaunchTensor>(x_dtype, y_dtype, a, flat, !whole, fast, static_cast<hipStream_t>(stream));

@@ -205,3 +205,12 @@ def test_fused_streams_envelope(n, k, qbn, inside):
     # default: the streaming kernel's envelope (bmm_fused_stream_ok)
     from practice_cuda_amd.impls.hip_per_block import fused_streams
     assert fused_streams(n, k, qbn) is inside
+
+
+def test_products_past_a_launch_are_refused():
+    """2^24 output tiles of 256 threads: a launch would run the remainder of 2^32 threads only."""
+    L = _lib.lib()
+    args = (FAKE, FAKE, _lib.E4M3FN, 2 ** 24, 1, 1, 17, 17, 17, 1, 17, 1, 17, FAKE, _lib.BF16, 1, 1, 1, None, 0, 0, 0, 0,
+            FAKE, 1, 1, 0, FAKE, 1, 1, 0, _lib.SCALE_CHANNEL, 0, 1, 128, 1, _lib.ACT_NONE, None)
+    assert L.pcamd_bmm_scaled(*args) == _lib.ERR_UNSUPPORTED
+    assert b"too many output tiles" in L.pcamd_last_error()
