@@ -1749,8 +1749,13 @@ extern "C" int pcamd_quant_block(const void* x, int x_dtype, int64_t batch, int6
     const int64_t units = flat ? (a.total + 127) / 128 : int64_t(batch) * m * a.segs;
     if (launchable((units + 3) / 4, kGroupThreads)) return dispatch_dt_fmt<LaunchGroups>(x_dtype, y_dtype, a, lpg, cpl, st);
   }
+  // (odd rows much shorter than a block leave most lanes of the tile kernel idle, in each of its passes
+  // over the block's rows: MI355X, bf16 [100000, n], element-wise / tiles, us: 16 x 512 blocks n = 33 18.1 / 20.0,
+  // 65 25.5 / 20.3; 128 x 128 n = 17 10.3 / 9.6 (300 rows 6.4 / 7.1), 33 level, 100 26.0 / 8.2 at 300 rows; 32 x 128
+  // n = 3 7.0 / 8.5, 9 8.8 / 8.2; 64 x 64 n = 3 5.3 / 6.0, 9 7.2 / 5.7)
   const int64_t lpr = block_n / 8;
-  if (rows && block_n >= 32 && lpr <= 64 && (block_m * lpr) % kThreads == 0 &&
+  const int64_t short_row = 4 * (block_m * lpr / kThreads) * std::max<int64_t>(1, block_n / 128);
+  if (rows && (fast || n > short_row) && block_n >= 32 && lpr <= 64 && (block_m * lpr) % kThreads == 0 &&
       block_m * lpr / kThreads <= kMaxSlots && batch * mb * nb < UINT32_MAX) {
     TileArgs a{};
     a.x = static_cast<const char*>(x); a.y = static_cast<uint8_t*>(y); a.scale = scale;
@@ -1885,6 +1890,15 @@ static ColParts col_parts(int64_t batch, int64_t m, int64_t n) {
   return {static_cast<int32_t>((slabs + per - 1) / per), static_cast<int32_t>(per * 128)};
 }
 
+// Per-column scales of few rows that are not whole aligned chunks: the
+// element-wise kernel (one launch, a workgroup per column) until its columns
+// take longer than the slab kernels' launches. MI355X, bf16, us, element-wise /
+// slabs: [256, 1031] 5.5 / 15.9, [1000, 1031] 15.3 / 16.6, [128, 4099] 8.6 / 11.5,
+// [256, 4099] 14.7 / 12.1, [1, 16383] 11.3 / 5.6, [256, 16383] 46.7 / 16.5.
+static bool few_odd_rows(int64_t batch, int64_t m, int64_t n) {
+  return m <= 1024 && batch * n <= (1 << 20) / std::max<int64_t>(m, 128);
+}
+
 static int quant_channel(const void* x, int x_dtype, int64_t batch, int64_t m, int64_t n,
                                    int64_t sxb, int64_t sxm, int64_t sxn, void* y, int y_dtype,
                                    int64_t syb, int64_t sym, int64_t syn, float* scale, int64_t ssb,
@@ -1941,7 +1955,7 @@ static int quant_channel(const void* x, int x_dtype, int64_t batch, int64_t m, i
     // Tall tensors: 128-row slabs in parallel (column maxima by atomic max in
     // the scale slots, then a quantize pass). Up to 256 rows one workgroup
     // per strip reads its rows twice.
-    if ((m > 256 || !fast) && launchable(a.strips, kThreads) && (m + 127) / 128 <= 65535 && batch <= 65535 &&
+    if ((fast ? m > 256 : !few_odd_rows(batch, m, n)) && launchable(a.strips, kThreads) && (m + 127) / 128 <= 65535 && batch <= 65535 &&
         launchable((batch * n + kThreads - 1) / kThreads, kThreads)) {
       if (workspace) {
         const ColParts p = col_parts(batch, m, n);
@@ -1974,6 +1988,7 @@ extern "C" int pcamd_quant_channel(const void* x, int x_dtype, int64_t batch, in
 
 extern "C" int64_t pcamd_quant_channel_workspace(int64_t batch, int64_t m, int64_t n, int channel_axis) {
   if (channel_axis != -1 || batch <= 0 || m <= 0 || n <= 0 || m > INT32_MAX) return 0;
+  if (m <= 256 && (n % 8 == 0 || few_odd_rows(batch, m, n))) return 0;
   return batch * col_parts(batch, m, n).parts * n * 4;
 }
 

@@ -59,11 +59,12 @@ def hip_per_channel_quant(
                                 dtype=torch.float32)
 
     L = _lib.lib()
-    # column maxima of the two-launch form (tall tensors); the caller's stream orders its reuse
+    # column maxima of tall tensors and of odd rows; the caller's stream orders its reuse
     ws, ws_bytes = None, 0
-    if channel_axis == -1 and m > 256:
+    if channel_axis == -1 and xs[2] == 1 and (m > 256 or n % 8):
         ws_bytes = L.pcamd_quant_channel_workspace(batch, m, n, channel_axis)
-        ws = torch.empty(ws_bytes, device=x.device, dtype=torch.uint8)
+        if ws_bytes:
+            ws = torch.empty(ws_bytes, device=x.device, dtype=torch.uint8)
     rc = _lib.launch(
         L.pcamd_quant_channel_ws, x,
         x.data_ptr(), _lib.dtype_code(x.dtype), batch, m, n, *xs,

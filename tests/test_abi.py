@@ -207,6 +207,14 @@ def test_fused_streams_envelope(n, k, qbn, inside):
     assert fused_streams(n, k, qbn) is inside
 
 
+def test_per_column_workspace_of_few_odd_rows():
+    """None where the element-wise kernel takes them in one launch."""
+    L = _lib.lib()
+    for m, n in ((1, 3), (64, 1001), (256, 1031), (128, 4099)):
+        assert L.pcamd_quant_channel_workspace(1, m, n, -1) == 0
+    assert L.pcamd_quant_channel_workspace(1, 200, 16383, -1) > 0
+
+
 def test_products_past_a_launch_are_refused():
     """2^24 output tiles of 256 threads: a launch would run the remainder of 2^32 threads only."""
     L = _lib.lib()

@@ -6,6 +6,7 @@ import pytest
 import torch
 
 from practice_cuda_amd import _lib
+from practice_cuda_amd.impls.hip_per_channel import hip_per_channel_quant
 
 pytestmark = pytest.mark.gpu
 
@@ -84,6 +85,18 @@ def test_per_column_workspace(dev, shape):
         torch.cuda.synchronize()
         got.append((y.view(torch.uint8), s.view(torch.int32)))
     assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
+
+
+@pytest.mark.parametrize("shape", [(1, 200, 1031), (1, 200, 4099), (1, 2, 16383), (3, 256, 2047)])
+def test_per_column_few_odd_rows(dev, shape):
+    """At most 256 odd rows: element-wise without a workspace, in slabs with one; same bytes as the aligned
+    columns of a wider tensor."""
+    b, m, n = shape
+    wide = _x((b, m, -(-n // 8) * 8), torch.bfloat16, dev)
+    x = wide[:, :, :n].contiguous()
+    r, w = hip_per_channel_quant(x, channel_axis=-1), hip_per_channel_quant(wide, channel_axis=-1)
+    assert torch.equal(r.tensor.view(torch.uint8), w.tensor.view(torch.uint8)[:, :, :n])
+    assert torch.equal(r.dequant_scale, w.dequant_scale[:, :n])
 
 
 def test_workspace_too_small(dev):
