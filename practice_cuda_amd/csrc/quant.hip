@@ -452,8 +452,9 @@ struct ColArgs {
   int32_t group_rows;     // rows per group (group mode)
   int32_t rpt;            // rows per thread (group mode) = group_rows / 16
   float fp8_max, eps;
-  float* parts;           // per-column scales, two-launch form: [batch, n_parts, n] maxima
+  float* parts;           // per-column scales with a workspace: [batch, n_parts, n] maxima
   int32_t n_parts, part_rows;
+  int32_t read_parts;     // of them the apply kernel takes: all, or the first after colchan_reduce_kernel
 };
 
 template <int DT, int FMT, bool CHANNEL>
@@ -1012,6 +1013,25 @@ __global__ __launch_bounds__(kThreads) void colchan_amax_kernel(ColArgs a) {
   }
 }
 
+// The maximum of each column's parts into its first part: 16 columns per
+// workgroup, 64 slices of the parts.
+constexpr int kReduceCols = 16, kReduceSlices = 64;
+__global__ __launch_bounds__(kReduceCols * kReduceSlices) void colchan_reduce_kernel(ColArgs a) {
+  __shared__ float red[kReduceSlices][kReduceCols];
+  const int lc = threadIdx.x % kReduceCols, slice = threadIdx.x / kReduceCols;
+  const int64_t c = int64_t(blockIdx.x) * kReduceCols + lc;
+  float* p = a.parts + int64_t(blockIdx.y) * a.n_parts * a.n + min(c, a.n - 1);
+  float mx = 0.0f;
+#pragma unroll 8
+  for (int i = slice; i < a.n_parts; i += kReduceSlices) mx = fmaxf(mx, p[i * a.n]);
+  red[slice][lc] = mx;
+  __syncthreads();
+  if (slice == 0 && c < a.n) {
+    for (int i = 1; i < kReduceSlices; ++i) mx = fmaxf(mx, red[i][lc]);
+    *p = mx;
+  }
+}
+
 // Same grid: quantize the slab with the finished column maxima.
 template <int DT, int FMT, bool NTS, bool UA, bool PARTS>
 __global__ __launch_bounds__(kThreads) void colchan_apply_kernel(ColArgs a) {
@@ -1033,22 +1053,35 @@ __global__ __launch_bounds__(kThreads) void colchan_apply_kernel(ColArgs a) {
   }
   // one division per column of the strip (lanes t < 128), shared through LDS
   __shared__ float qsv[128];
-  if (t < 128) {
-    const int64_t c = strip * 128 + t;
-    if constexpr (PARTS) {
-      float mx = 0.0f;
-      const float* p = a.parts + b * a.n_parts * a.n + min(c, a.n - 1);
-      int i = 0;
-      for (; i + 4 <= a.n_parts; i += 4)
-        mx = fmaxf(mx, fmaxf(fmaxf(p[i * a.n], p[(i + 1) * a.n]), fmaxf(p[(i + 2) * a.n], p[(i + 3) * a.n])));
-      for (; i < a.n_parts; ++i) mx = fmaxf(mx, p[i * a.n]);
+  if constexpr (PARTS) {
+    // few parts: the first half of the workgroup reads them; more: every second one per half.
+    // (Four loads in flight: eight take 16 more registers and two of seven waves per SIMD.)
+    __shared__ float pmax[2][128];
+    const bool halves = a.read_parts > 16;
+    const int64_t c = strip * 128 + (t & 127);
+    float mx = 0.0f;
+    if (halves || t < 128) {
+      const int64_t pitch = halves ? 2 * a.n : a.n;
+      const float* p = a.parts + b * a.n_parts * a.n + (t >> 7) * a.n + min(c, a.n - 1);
+      int left = halves ? (a.read_parts + 1 - (t >> 7)) >> 1 : a.read_parts;
+      for (; left >= 4; left -= 4, p += 4 * pitch)
+        mx = fmaxf(mx, fmaxf(fmaxf(p[0], p[pitch]), fmaxf(p[2 * pitch], p[3 * pitch])));
+      for (; left > 0; --left, p += pitch) mx = fmaxf(mx, *p);
+    }
+    if (halves) {
+      pmax[t >> 7][t & 127] = mx;
+      __syncthreads();
+      mx = fmaxf(pmax[0][t & 127], pmax[1][t & 127]);
+    }
+    if (t < 128) {
       const Scales sc = channel_scales(mx, a.fp8_max, a.eps);
       qsv[t] = sc.qs;
       if (blockIdx.y == 0 && c < a.n) a.scale[b * a.ssb + c * a.ssn] = sc.ds;
-    } else {
-      const uint32_t* amax_bits = reinterpret_cast<const uint32_t*>(a.scale) + b * a.ssb;
-      qsv[t] = c < a.n ? channel_scales(__uint_as_float(amax_bits[c * a.ssn]), a.fp8_max, a.eps).qs : 0.0f;
     }
+  } else if (t < 128) {
+    const int64_t c = strip * 128 + t;
+    const uint32_t* amax_bits = reinterpret_cast<const uint32_t*>(a.scale) + b * a.ssb;
+    qsv[t] = c < a.n ? channel_scales(__uint_as_float(amax_bits[c * a.ssn]), a.fp8_max, a.eps).qs : 0.0f;
   }
   __syncthreads();
   float qs[8];
@@ -1592,6 +1625,10 @@ struct LaunchColChan {
     if (a.parts != nullptr) {
       const dim3 pgrid(grid.x, static_cast<uint32_t>(a.n_parts), grid.z);
       colchan_amax_kernel<DT, UA, true><<<pgrid, kThreads, 0, st>>>(a);
+      if (a.read_parts < a.n_parts) {
+        const dim3 rgrid(static_cast<uint32_t>((a.n + kReduceCols - 1) / kReduceCols), grid.z);
+        colchan_reduce_kernel<<<rgrid, kReduceCols * kReduceSlices, 0, st>>>(a);
+      }
       colchan_apply_kernel<DT, FMT, NTS, UA, true><<<grid, kThreads, 0, st>>>(a);
       return check_launch("per-column kernels");
     }
@@ -1880,14 +1917,22 @@ extern "C" int pcamd_quant_block_dual_ex(const void* x, int x_dtype, int64_t bat
                                 eps, stream);
 }
 
-// Rows per part of the two-launch per-column form: about 1024 workgroups for
-// the amax pass, 8 to 32 parts per column (the apply pass reads them all).
-struct ColParts { int32_t parts, rows; };
+// Rows per part of the per-column scales with a workspace: about 1024 workgroups
+// for the amax pass. Up to 64 parts per column the apply pass reads them all
+// (two launches); a tall, narrow tensor whose parts would then be longer than
+// three slabs takes at least twice as many, reduced to one in a third launch.
+// MI355X, us of GPU time with the input in cache / from HBM, four launches with
+// atomic maxima -> this: bf16 [65536, 256] 22.5 / 25.6 -> 15.1 / 17.1, fp32 36.6 /
+// 36.9 -> 29.0 / 29.0, bf16 [300000, 64] 61.3 / 62.2 -> 26.8 / 27.0, [20000, 1024]
+// 21.1 / 21.6 -> 17.4 / 17.8 (reduced: 22.0 / 20.7), [8192, 256] 10.7 / 11.9 -> 8.2 / 9.2.
+struct ColParts { int32_t parts, rows; bool reduce; };
 static ColParts col_parts(int64_t batch, int64_t m, int64_t n) {
-  const int64_t slabs = (m + 127) / 128, wgs = (n + 127) / 128 * batch;
-  const int64_t want = std::min<int64_t>(slabs, std::min<int64_t>(32, std::max<int64_t>(8, (1023 + wgs) / wgs)));
+  const int64_t slabs = (m + 127) / 128, wgs = (n + 127) / 128 * batch, full = (1023 + wgs) / wgs;
+  int64_t want = std::min<int64_t>(slabs, std::min<int64_t>(64, std::max<int64_t>(8, full)));
+  const bool reduce = full >= 2 * want && slabs > 3 * want;
+  if (reduce) want = std::min(slabs, full);
   const int64_t per = (slabs + want - 1) / want;
-  return {static_cast<int32_t>((slabs + per - 1) / per), static_cast<int32_t>(per * 128)};
+  return {static_cast<int32_t>((slabs + per - 1) / per), static_cast<int32_t>(per * 128), reduce};
 }
 
 // Per-column scales of few rows that are not whole aligned chunks: the
@@ -1963,6 +2008,7 @@ static int quant_channel(const void* x, int x_dtype, int64_t batch, int64_t m, i
           return set_error(PCAMD_ERR_INVALID, "the workspace must hold %lld bytes (pcamd_quant_channel_workspace)",
                            (long long)(batch * p.parts * n * 4));
         a.parts = workspace; a.n_parts = p.parts; a.part_rows = p.rows;
+        a.read_parts = p.reduce ? 1 : p.parts;
       }
       return dispatch_dt_fmt<LaunchColChan>(x_dtype, y_dtype, a, batch, !fast, st);
     }

@@ -207,6 +207,17 @@ def test_fused_streams_envelope(n, k, qbn, inside):
     assert fused_streams(n, k, qbn) is inside
 
 
+def test_per_column_workspace_of_tall_tensors():
+    """Maxima per column and part: at least 512 workgroups' worth of parts however
+    narrow the tensor is, at most one part per 128 rows."""
+    L = _lib.lib()
+    for batch, m, n in ((1, 65536, 256), (1, 131072, 128), (1, 300000, 64), (8, 16384, 128), (1, 32768, 1536),
+                        (1, 4096, 14336), (1, 65536, 900)):
+        parts, rest = divmod(L.pcamd_quant_channel_workspace(batch, m, n, -1), 4 * batch * n)
+        assert rest == 0 and 1 <= parts <= -(-m // 128)
+        assert parts * batch * -(-n // 128) >= 512, (batch, m, n, parts)
+
+
 def test_per_column_workspace_of_few_odd_rows():
     """None where the element-wise kernel takes them in one launch."""
     L = _lib.lib()

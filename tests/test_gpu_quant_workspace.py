@@ -87,6 +87,27 @@ def test_per_column_workspace(dev, shape):
     assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
 
 
+@pytest.mark.parametrize("shape", [(1, 24578, 130), (1, 30000, 8), (2, 25000, 3), (1, 70000, 264)])
+def test_per_column_workspace_tall(dev, shape):
+    """Tall, narrow tensors: more than 64 parts per column, reduced to one before the quantize pass."""
+    x = _x(shape, torch.bfloat16, dev)
+    b, m, n = shape
+    L, st = _lib.lib(), _lib.stream_of(x)
+    size = L.pcamd_quant_channel_workspace(b, m, n, -1)
+    assert size > 64 * b * n * 4
+    got = []
+    for ws in (None, torch.full((size // 4 + 16,), float("nan"), device=dev)):
+        y = torch.zeros(shape, dtype=torch.float8_e4m3fn, device=dev)
+        s = torch.zeros(b, n, device=dev)
+        rc = L.pcamd_quant_channel_ws(*_head(x, y), s.data_ptr(), n, 1, -1, 448.0, 1e-12, _lib.ptr(ws),
+                                      0 if ws is None else size, st)
+        _lib.check(rc, "per-column")
+        torch.cuda.synchronize()
+        assert ws is None or torch.isnan(ws[size // 4:]).all()
+        got.append((y.view(torch.uint8), s.view(torch.int32)))
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
+
+
 @pytest.mark.parametrize("shape", [(1, 200, 1031), (1, 200, 4099), (1, 2, 16383), (3, 256, 2047)])
 def test_per_column_few_odd_rows(dev, shape):
     """At most 256 odd rows: element-wise without a workspace, in slabs with one; same bytes as the aligned
