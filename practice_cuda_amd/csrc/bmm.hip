@@ -517,10 +517,14 @@ static int bmm_scaled(const void* a, int a_fmt, const void* b, int b_fmt, int64_
 
   // tuned path: K a multiple of 128, 16-byte aligned operands and rows,
   // power-of-two block sizes, 32-bit addressable batch slices.
-  // PCAMD_BMM_WIDE=0 / PCAMD_BMM_STREAM=0 / PCAMD_BMM_GENERIC select the other
-  // kernels (read once)
+  // PCAMD_BMM_WIDE=0 / PCAMD_BMM_STREAM=0 / PCAMD_BMM_SPLIT=0 / PCAMD_BMM_GENERIC
+  // select the other kernels (read once)
   static const bool env_no_wide = [] {
     const char* e = getenv("PCAMD_BMM_WIDE");
+    return e && e[0] == '0';
+  }();
+  static const bool env_no_split = [] {
+    const char* e = getenv("PCAMD_BMM_SPLIT");
     return e && e[0] == '0';
   }();
   static const bool env_generic = getenv("PCAMD_BMM_GENERIC") != nullptr;
@@ -581,8 +585,9 @@ static int bmm_scaled(const void* a, int a_fmt, const void* b, int b_fmt, int64_
           bmm_stream_ok(f, a_k, b_k, fmode, batch, args.qbm, args.qbn, ssa1, ssb2))
         return bmm_stream_launch(f, a_fmt, batch, st);
       // products of several K steps on a short grid, and unaligned operands
-      if (bmm_split_ok(f, a_fmt, b_fmt, a_k, b_k, fmode, batch, st) &&
-          (!fast || (wide && bmm_split_pays(f, batch, st))))
+      if (!env_no_split && bmm_split_ok(f, a_fmt, b_fmt, a_k, b_k, fmode, batch, st) &&
+          (fast ? wide && bmm_split_pays(f, a_k, b_k, fmode, batch, st)
+                : bmm_split_over_general(f, a_k, b_k, fmode, args.vec_a && args.vec_b, batch, st)))
         return bmm_split_launch(f, a_k, b_k, fmode, batch, st);
       if (tm * tn * batch > UINT32_MAX / 512) return launch_general();
       if (fast && wide) return bmm_wide_launch(f, a_fmt, b_fmt, a_k, b_k, fmode, st);

@@ -72,12 +72,17 @@ int bmm_wide_tile();
 
 // K-split kernel (bmm_split.h): small grids, and operands of any alignment
 // (no row of them 16-byte aligned, K any size). bmm_split_ok is its envelope:
-// e4m3fn operands, quant-K 128 in block mode, rows of at least 16 bytes;
-// bmm_split_pays whether it is ahead of the tiled kernels on operands that
-// those take too. It uses a's strides, extents and sizes, not its tile counts.
+// e4m3fn operands, quant-K 128 in block mode, rows of at least 16 bytes, a
+// grid that one launch takes; bmm_split_pays whether it is ahead of the tiled
+// kernels on operands that those take too, bmm_split_over_general whether it
+// is ahead of the general kernel on the others (aligned_rows: both operands'
+// rows are 16-byte aligned). It uses a's strides, extents and sizes, not its
+// tile counts.
 bool bmm_split_ok(const FastArgs& a, int a_fmt, int b_fmt, bool a_k, bool b_k, int mode, int64_t batch,
                   hipStream_t st);
-bool bmm_split_pays(const FastArgs& a, int64_t batch, hipStream_t st);
+bool bmm_split_pays(const FastArgs& a, bool a_k, bool b_k, int mode, int64_t batch, hipStream_t st);
+bool bmm_split_over_general(const FastArgs& a, bool a_k, bool b_k, int mode, bool aligned_rows, int64_t batch,
+                            hipStream_t st);
 int bmm_split_launch(const FastArgs& a, bool a_k, bool b_k, int mode, int64_t batch, hipStream_t st);
 
 }  // namespace pcamd

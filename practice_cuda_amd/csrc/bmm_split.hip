@@ -42,6 +42,15 @@ inline Shape pick(const FastArgs& a, int64_t batch, int cus, bool block) {
   return block ? k1x4w4 : k1x4w8;
 }
 
+// whether the tiled kernels store a's output through LDS (their epilogue's
+// conditions, bmm_wide.h)
+inline bool staged_output(const FastArgs& a) {
+  const bool bias16 = (a.bias_dtype == kBF16 || a.bias_dtype == kF16) && a.sbiasn == 1 && a.sbiasm % 4 == 0 &&
+                      a.sbiasb % 4 == 0 && (reinterpret_cast<uintptr_t>(a.bias) & 7) == 0;
+  return (a.c_dtype == kBF16 || a.c_dtype == kF16) && (a.bias == nullptr || bias16) && a.n % 8 == 0 &&
+         a.scm % 8 == 0 && a.scb % 8 == 0 && (reinterpret_cast<uintptr_t>(a.c) & 15) == 0;
+}
+
 template <bool A_K, bool B_K, int MODE>
 int launch_shape(const FastArgs& a, int64_t batch, hipStream_t st) {
   constexpr bool BLOCK = MODE == 0;
@@ -90,15 +99,44 @@ bool bmm_split_ok(const FastArgs& a, int a_fmt, int b_fmt, bool a_k, bool b_k, i
   return true;
 }
 
-// Up to two 64 x 64 tiles per CU the K-split kernel is ahead of the tiled
-// ones, whose few workgroups then walk K one step after the other (MI355X,
-// block scales, tiled -> here, us: 16 x 14336 x 4096 50.1 -> 15.1, 16 x 1024 x
-// 1024 9.9 -> 3.5, 128 x 14336 x 4096 52.3 -> 35.6, 512 x 1024 x 4096 40.3 ->
-// 15.5, 512 x 4096 x 1024 12.9 -> 11.1); at four (4096 x 1024 x 512: 8.9 ->
-// 13.9) it is behind: each operand byte is loaded for 64 outputs instead of
-// 128 or 256.
-bool bmm_split_pays(const FastArgs& a, int64_t batch, hipStream_t st) {
-  return bmmp::tiles(a, batch, 64, 64) <= 2 * int64_t(device_cu_count(st));
+// Up to one 64 x 64 tile per CU the K-split kernel is ahead of the tiled ones,
+// whose workgroups then walk K one step after the other on part of the chip;
+// beyond, each operand byte is loaded for 64 outputs instead of 128. With two
+// K steps there is little to split: the line is lower where the waves' sums
+// meet once (channel, tensor). From 32 steps on it pays up to two tiles per CU
+// when the weight comes from HBM, except where the operands' majors differ in
+// block mode; so it does with at most 32 rows (smaller tiles here, padding
+// there) and with outputs that the tiled kernels store element by element.
+// MI355X, us with the operands in L2 / from HBM, tiled (128 x 128
+// tiles) -> here, block scales and N-major B unless said:
+//   16 x 14336 x 4096   30.6 / 40.2 -> 17.1 / 21.0
+//   256 x 2048 x 1024    8.3 / 10.5 ->  5.8 /  6.0
+//   1024 x 1024 x 256    4.7 /  5.2 ->  4.8 /  4.8   (one tile per CU; tensor 6.0 / 6.3 -> 7.0 / 6.9)
+//   512 x 2048 x 4096   22.9 / 41.0 -> 19.1 / 23.3
+//   128 x 14336 x 1024   8.6 / 14.8 -> 17.5 / 19.5   (1.75 per CU; K-major B 8.3 / 12.8 -> 10.9 / 12.9)
+//   512 x 4096 x 4096   29.3 / 40.4 -> 52.8 / 58.4   (two; K-major B 28.2 / 37.6 -> 31.9 / 33.6,
+//                       channel, K-major B 24.7 / 34.5 -> 28.5 / 28.3)
+//   512 x 4096 x 256, fp32 output 21.8 -> 11.1, fp8 26.3 -> 9.3; 512 x (16 x 64 x 256) 17.1 -> 4.1
+bool bmm_split_pays(const FastArgs& a, bool a_k, bool b_k, int mode, int64_t batch, hipStream_t st) {
+  const int64_t t = bmmp::tiles(a, batch, 64, 64), cus = device_cu_count(st);
+  const bool deep = a.k >= 32 * bmmp::BK && (mode != 0 || a_k == b_k);
+  if (deep || a.m <= 32 || !bmmp::staged_output(a)) return t <= 2 * cus;
+  return mode != 0 && a.k <= 2 * bmmp::BK ? 4 * t <= 3 * cus : t <= cus;
+}
+
+// Operands that the tiled kernels do not take: the general kernel is slower
+// wherever it gathers bytes (rows not 16-byte aligned), folds block scales, or
+// has few of its 128 x 128 tiles. On aligned rows (K no multiple of 4, or
+// ragged and below 128) and more than six 64 x 64 tiles per CU it is ahead
+// with one scale, and with channel scales over eight or more K steps unless
+// both operands are K-major. MI355X, us, general / here, MN-major operands:
+// tensor 4096 x 4096 x 1031 86.8 / 129, 2048 x 3072 x 1031 46.6 / 49.1, 2048 x 2048 x
+// 1031 35.6 / 32.8, 8192 x 8192 x 64 182 / 250; channel 4096 x 4096 x 1031 138 / 155
+// (K-major 1.00 : 0.89), 4096 x 4096 x 515 1 : 0.9; block 4096 x 4096 x 1031 205 / 95.
+bool bmm_split_over_general(const FastArgs& a, bool a_k, bool b_k, int mode, bool aligned_rows, int64_t batch,
+                            hipStream_t st) {
+  if (!aligned_rows || mode == 0 || bmmp::tiles(a, batch, 64, 64) <= 6 * int64_t(device_cu_count(st))) return true;
+  return mode == 1 && ((a_k && b_k) || a.k < 8 * bmmp::BK);
 }
 
 int bmm_split_launch(const FastArgs& a, bool a_k, bool b_k, int mode, int64_t batch, hipStream_t st) {
