@@ -527,6 +527,10 @@ static int bmm_scaled(const void* a, int a_fmt, const void* b, int b_fmt, int64_
     const char* e = getenv("PCAMD_BMM_SPLIT");
     return e && e[0] == '0';
   }();
+  static const bool env_whole_tiles = [] {  // bmm_wide.h reads it too
+    const char* e = getenv("PCAMD_BMM_HALVES");
+    return e && e[0] == '0';
+  }();
   static const bool env_generic = getenv("PCAMD_BMM_GENERIC") != nullptr;
   static const bool env_no_stream = [] {
     const char* e = getenv("PCAMD_BMM_STREAM");
@@ -586,7 +590,7 @@ static int bmm_scaled(const void* a, int a_fmt, const void* b, int b_fmt, int64_
         return bmm_stream_launch(f, a_fmt, batch, st);
       // products of several K steps on a short grid, and unaligned operands
       if (!env_no_split && bmm_split_ok(f, a_fmt, b_fmt, a_k, b_k, fmode, batch, st) &&
-          (fast ? wide && bmm_split_pays(f, a_k, b_k, fmode, batch, st)
+          (fast ? wide && !env_whole_tiles && bmm_split_pays(f, a_k, b_k, fmode, batch, st)
                 : bmm_split_over_general(f, a_k, b_k, fmode, args.vec_a && args.vec_b, batch, st)))
         return bmm_split_launch(f, a_k, b_k, fmode, batch, st);
       if (tm * tn * batch > UINT32_MAX / 512) return launch_general();

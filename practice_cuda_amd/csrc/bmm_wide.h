@@ -326,9 +326,9 @@ __global__ __launch_bounds__(Geom<SMALL>::NT, SMALL ? 2 : 1) void bmm_wide_kerne
     if constexpr (B_K) return frag_k(stage + A_BYTES, wcol + j * 16 + lr, lg);
     else return frag_mn<BN>(stage + A_BYTES, wcol + j * 16, lane);
   };
-  // Block scales of K step ks for this thread's slot: waves 0-3 fetch the
-  // tile's 256 row scales, waves 4-7 its 256 column scales (the wave index is
-  // made scalar so the choice is uniform). Rows / columns past the matrix read
+  // Block scales of K step ks for this thread's slot: the first half of the
+  // waves fetch the tile's row scales, the others its column scales (the wave
+  // index is made scalar so the choice is uniform). Rows / columns past the matrix read
   // the last valid scale; they only feed outputs that are never stored.
   const bool row_scales = wave < WAVES / 2;
   const int slot = t & (BM - 1);
@@ -752,6 +752,15 @@ inline bool transposed_disabled() {
   return off;
 }
 
+// PCAMD_BMM_HALVES=0 keeps 256 x 256 tiles on grids that leave CUs idle (read once)
+inline bool short_grids_disabled() {
+  static const bool off = [] {
+    const char* e = getenv("PCAMD_BMM_HALVES");
+    return e && e[0] == '0';
+  }();
+  return off;
+}
+
 template <bool A_K, bool B_K, int FA, int FB, int MODE, int SBK, int JN, bool KT, bool CT = false, bool SMALL = false>
 int launch_tiles(const FastArgs& a, int grid, hipStream_t st) {
   constexpr int NT = Geom<SMALL>::NT, LDS_BYTES = Geom<SMALL>::LDS_BYTES;
@@ -807,7 +816,7 @@ template <bool A_K, bool B_K, int FA, int FB, int MODE, int SBK, bool KT>
 int launch_one(const FastArgs& a, hipStream_t st) {
   const int cus = device_cu_count(st);
   const int64_t batch = a.total_tiles / a.tiles_per_batch;
-  if (cus > 0) {
+  if (cus > 0 && !short_grids_disabled()) {
     const int64_t small = tiles_of(a, batch, Geom<true>::BM, Geom<true>::BN);
     if (small <= UINT32_MAX / Geom<true>::NT && small_cost(small, a.k, cus) < tile_waves(a.total_tiles, cus)) {
       const FastArgs t = with_tiles(a, batch, Geom<true>::BM, Geom<true>::BN);

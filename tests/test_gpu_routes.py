@@ -61,7 +61,7 @@ def test_short_grid_rule_element_wise_outputs(dev):
     assert not same_bits_as_tiled(32, 2 * _columns(dev, 2), 1024, dev)
 
 
-@pytest.mark.parametrize("switch", ["PCAMD_BMM_SPLIT"])
+@pytest.mark.parametrize("switch", ["PCAMD_BMM_SPLIT", "PCAMD_BMM_HALVES"])
 def test_switches_keep_short_grids_on_tiles(dev, switch):
     """Each is read once per process, so it runs in one of its own."""
     assert not same_bits_as_tiled(64, 512, 1024, dev)
