@@ -17,8 +17,8 @@ from practice_cuda_amd.registry import QuantResult
 pytestmark = pytest.mark.gpu
 E4M3 = torch.float8_e4m3fn
 
-# grids past the K-split kernel's: whole tiles with a short last wave (half
-# tiles), 128 x 128 tiles; partial tiles in both directions
+# 128 x 128 tiles (first and last) and whole tiles, partial ones in both
+# directions (half tiles: test_gpu_tiles.py)
 SHAPES = [(1, 1000, 2056, 160), (3, 1030, 8200, 256), (2, 512, 8192, 144)]
 
 

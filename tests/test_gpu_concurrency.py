@@ -38,7 +38,7 @@ def _inputs(dev, seed):
 
 def _run(x, w, a4, b4):
     """Quantizers (row groups, per-row channel, 128x128 tiles, the dual
-    kernel), the wide BMM (K = 1024), the streaming BMM (K = 128, N = 512)
+    kernel), the K-split BMM (K = 1024), the streaming BMM (K = 128, N = 512)
     and the fused activation-quant BMM (N = 128, K = 1024: its streaming
     kernel)."""
     qx = hip_per_block_quant(x[None], block_m=1, block_n=128)
@@ -66,10 +66,26 @@ def _bits(t):
                                                                     else torch.int32)
 
 
-def test_threads_on_separate_streams_match_serial(dev):
+def _wide_inputs(dev, seed):
+    g = torch.Generator(device=dev).manual_seed(seed)
+    return (torch.randn(1, 2304, 512, generator=g, device=dev).bfloat16(),
+            torch.randn(1, 512, 2048, generator=g, device=dev).bfloat16(),
+            torch.randn(1, 9000, 1031, generator=g, device=dev).bfloat16())
+
+
+def _run_wide(a, b, x):
+    """The wide BMM (a grid past the K-split kernel's) and the column quantizers that take a workspace: the
+    operand's, and odd rows."""
+    qa, qb = hip_per_block_quant(a, block_m=1, block_n=128), hip_per_block_quant(b, block_m=128, block_n=128)
+    qc, qx = hip_per_channel_quant(a, channel_axis=-1), hip_per_channel_quant(x, channel_axis=-1)
+    return [hip_per_block_bmm(qa, qb), qc.tensor, qc.dequant_scale, qx.tensor, qx.dequant_scale]
+
+
+@pytest.mark.parametrize("make,run", [(_inputs, _run), (_wide_inputs, _run_wide)], ids=["short", "wide"])
+def test_threads_on_separate_streams_match_serial(dev, make, run):
     print(f"concurrency: {THREADS} threads x {ITERS} iterations", flush=True)
-    inputs = [_inputs(dev, 100 + i) for i in range(THREADS)]
-    expected = [[_bits(t).clone() for t in _run(*inp)] for inp in inputs]
+    inputs = [make(dev, 100 + i) for i in range(THREADS)]
+    expected = [[_bits(t).clone() for t in run(*inp)] for inp in inputs]
     torch.cuda.synchronize()
     results = [None] * THREADS
     errors = []
@@ -82,7 +98,7 @@ def test_threads_on_separate_streams_match_serial(dev):
             with torch.cuda.stream(s):
                 out = None
                 for _ in range(ITERS):
-                    out = _run(*inputs[i])
+                    out = run(*inputs[i])
                 results[i] = [_bits(t) for t in out]
             s.synchronize()
         except Exception as exc:  # surfaced below, with the thread's index

@@ -144,10 +144,10 @@ def _bmm_abi(a, b, c, sa, sb, mode, saq):
     torch.cuda.synchronize()
 
 
-# (batch, m, n, k): K = 128 takes the single-step kernel, K = 512 the wide
-# kernel, the odd shape the general kernel
-KERNEL_SHAPES = {"single_k128": (2, 256, 384, 128), "wide_k512": (2, 512, 512, 512),
-                 "general_unaligned": (2, 33, 47, 200)}
+# (batch, m, n, k): K = 128 takes the single-step kernel, the others the K-split
+# kernel (test_gpu_tiles.py has the wide and general ones)
+KERNEL_SHAPES = {"single_k128": (2, 256, 384, 128), "split_k512": (2, 512, 512, 512),
+                 "split_unaligned": (2, 33, 47, 200)}
 
 
 @pytest.mark.parametrize("out", ["f32", "bf16"])
@@ -155,7 +155,7 @@ KERNEL_SHAPES = {"single_k128": (2, 256, 384, 128), "wide_k512": (2, 512, 512, 5
 @pytest.mark.parametrize("kernel", sorted(KERNEL_SHAPES))
 def test_scales_are_quant(dev, kernel, mode, out):
     """fp32 output goes through the per-element epilogue, bf16 output (aligned
-    shapes) through the LDS-staged one of the single-step and wide kernels."""
+    shapes) through the LDS-staged one of the single-step kernel."""
     bsz, m, n, k = KERNEL_SHAPES[kernel]
     print(f"scales_are_quant {kernel} {mode} {out}", flush=True)
     odt = torch.float32 if out == "f32" else torch.bfloat16

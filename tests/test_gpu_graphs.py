@@ -10,7 +10,7 @@ import torch
 from practice_cuda_amd.impls.hip_per_block import (hip_per_block_bmm, hip_per_block_bmm_quant_a,
                                                    hip_per_block_quant, hip_per_block_quant_dual)
 from practice_cuda_amd.impls.hip_per_channel import hip_per_channel_quant
-from practice_cuda_amd.impls.hip_per_tensor import hip_per_tensor_quant
+from practice_cuda_amd.impls.hip_per_tensor import hip_per_tensor_bmm, hip_per_tensor_quant
 
 pytestmark = pytest.mark.gpu
 
@@ -86,7 +86,7 @@ def test_bmm_replay(dev):
     b1 = torch.randn(4, 128, 256, generator=g).bfloat16().to(dev)
     qa1 = hip_per_block_quant(a1, block_m=1, block_n=128)
     qb1 = hip_per_block_quant(b1, block_m=128, block_n=128)
-    a2 = torch.randn(1, 33, 256, generator=g).bfloat16().to(dev)  # ragged M / N: general kernel
+    a2 = torch.randn(1, 33, 256, generator=g).bfloat16().to(dev)  # ragged M / N
     b2 = torch.randn(1, 256, 47, generator=g).bfloat16().to(dev)
     qa2 = hip_per_block_quant(a2, block_m=1, block_n=128)
     qb2 = hip_per_block_quant(b2, block_m=128, block_n=128)
@@ -101,16 +101,37 @@ def test_bmm_replay(dev):
     bias5 = torch.randn(2, 512, 192, generator=g).bfloat16().to(dev)
     bias_w = torch.randn(2, 512, 384, generator=g).bfloat16().to(dev)
     fns = {
-        "wide": lambda: hip_per_block_bmm(qa, qb),
+        "split": lambda: hip_per_block_bmm(qa, qb),
         "single": lambda: hip_per_block_bmm(qa1, qb1),
-        "general": lambda: hip_per_block_bmm(qa2, qb2),
+        "split_ragged": lambda: hip_per_block_bmm(qa2, qb2),
         "fused_stream_n128": lambda: hip_per_block_bmm_quant_a(ah, qb3, return_quant=True),
         "fused_stream_n256": lambda: hip_per_block_bmm_quant_a(ah, qb4),
         "fused_tiled": lambda: hip_per_block_bmm_quant_a(ah, qb, always_fused=True),
         # epilogues: 16-bit bias + GELU (8-byte loads and stores), fp32 output
-        # (per-element), and the wide GEMM's LDS-staged bias + GELU
+        # (per-element)
         "fused_stream_n192_bias_gelu": lambda: hip_per_block_bmm_quant_a(ah, qb5, bias=bias5, activation="gelu"),
         "fused_stream_n64_f32": lambda: hip_per_block_bmm_quant_a(ah, qb6, out_dtype=torch.float32),
-        "wide_bias_gelu": lambda: hip_per_block_bmm(qa, qb, bias=bias_w, activation="gelu"),
+        "split_bias_gelu": lambda: hip_per_block_bmm(qa, qb, bias=bias_w, activation="gelu"),
+    }
+    _replay_matches_eager(dev, fns)
+
+
+def test_tiled_bmm_replay(dev):
+    """Grids past the K-split kernel's (two 64 x 64 tiles per CU): 128 x 128 tiles, whole ones with half tiles
+    behind them (two launches) and LDS-staged bias + GELU; and the general kernel (e5m2, unaligned rows)."""
+    cus = torch.cuda.get_device_properties(dev).multi_processor_count
+    g = torch.Generator(device=dev).manual_seed(9)
+    a = torch.randn(1, (2 * cus + cus // 8) // 16 * 256, 256, generator=g, device=dev).bfloat16()
+    b = torch.randn(1, 256, 4096, generator=g, device=dev).bfloat16()
+    bias = torch.randn(1, 1, 4096, generator=g, device=dev).bfloat16()
+    qb = hip_per_block_quant(b, block_m=128, block_n=128)
+    small, large = (hip_per_block_quant(a[:, :m], block_m=1, block_n=128) for m in (cus * 4 + 80, a.shape[1]))
+    u, v = (hip_per_tensor_quant(t.contiguous(), fp8_dtype=torch.float8_e5m2) for t in (a[:, :33, :201], b[:, :201, :47]))
+    fns = {
+        "small_tiles": lambda: hip_per_block_bmm(small, qb),
+        "small_tiles_bias_gelu": lambda: hip_per_block_bmm(small, qb, bias=bias.expand(-1, cus * 4 + 80, -1),
+                                                           activation="gelu"),
+        "half_tiles": lambda: hip_per_block_bmm(large, qb, out_dtype=torch.float16),
+        "general": lambda: hip_per_tensor_bmm(u, v),
     }
     _replay_matches_eager(dev, fns)

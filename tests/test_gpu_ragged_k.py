@@ -1,5 +1,8 @@
 """GPU parity of the scaled FP8 BMM when K is not a multiple of 128.
 
+(Most shapes here are short grids, which run on the K-split kernel; the wide
+kernel's tile forms are in test_gpu_tiles.py.)
+
 The wide kernel takes K > 128 with K % 4 == 0: its last K step holds fewer
 than 128 valid k, and the fragment words past them are zeroed in both
 operands (a K-major row's tail holds the next row's bytes). The reference's
@@ -143,10 +146,10 @@ def test_legacy_fp16_bias_published_shapes(dev, shape, b_k_major):
 
 @pytest.mark.parametrize("layout", ["a_k_b_k", "a_k_b_n"])
 def test_ragged_k_tail_bytes_are_masked(dev, layout):
-    """K-major rows stored with a padded pitch (1024 bytes for K = 960): the
-    last K step reads each row's 64 padding bytes, which hold NaN codes
-    (0x7F) here. The masked words never reach the MFMA, so the output equals
-    the product of the same values stored unpadded, bit for bit."""
+    """K-major rows stored with a padded pitch (1024 bytes for K = 960) whose
+    padding holds NaN codes (0x7F): a short grid, so the K-split kernel, whose
+    loads end with the row. The output equals the product of the same values
+    stored unpadded, bit for bit."""
     bsz, m, n, k, pitch = 2, 256, 256, 960, 1024
     print(f"ragged K NaN padding {layout}", flush=True)
     a, b = _fp8((bsz, m, k), 41), _fp8((bsz, k, n), 42)

@@ -2,7 +2,9 @@
 
 When the last wave of 256 x 256 tiles would fill at most half the CUs, those
 tiles run in a second launch as 256 x 128 halves, two workgroups per tile, so
-that the partial wave still occupies every CU. Shapes here are sized from the
+that the partial wave still occupies every CU; with one whole wave before it and
+K <= 2048, 128 x 128 tiles fill the chip better and run instead (the halves behind
+two waves are in test_gpu_tiles.py). Shapes here are sized from the
 device's CU count so that the tile count is CUs + a small tail, and cover:
 - even and odd numbers of K steps;
 - K-major and MN-major operands, and one scale per column of B (128 x 1
