@@ -40,14 +40,13 @@ SETTLE_MS = 100.0            # untimed load before the first (headline) measurem
 # committed counter summary (profiles/pmc_bmm.json) to the code that runs now
 CONFIG4_KERNEL = "pcamd::bmms::bmm_stream_kernel<3>"
 # template arguments: A K-major, B K-major, A / B fp8 formats, scale mode, B-scale kind,
-# sub-tiles per wave, ragged K, transposed output (wgrad: 256 x 224 tiles of C^T)
-# (as profiled; the kernel has since gained a tenth argument, false for these
-# instantiations, whose code is unchanged)
-CONFIG5_KERNELS = {"fwd_a_k_b_k": ("fwd", ["pcamd::bmmw::bmm_wide_kernel<true, true, 3, 3, 0, 0, 8, false, false>"]),
+# sub-tiles per wave, ragged K, transposed output (wgrad: 256 x 224 tiles of C^T), 128 x 128 tiles
+CONFIG5_KERNELS = {"fwd_a_k_b_k": ("fwd",
+                                   ["pcamd::bmmw::bmm_wide_kernel<true, true, 3, 3, 0, 0, 8, false, false, false>"]),
                    "dgrad_a_k_b_n": ("dgrad",
-                                     ["pcamd::bmmw::bmm_wide_kernel<true, false, 3, 3, 0, 0, 8, false, false>"]),
+                                     ["pcamd::bmmw::bmm_wide_kernel<true, false, 3, 3, 0, 0, 8, false, false, false>"]),
                    "wgrad_a_m_b_n": ("wgrad_a_m_b_n",
-                                     ["pcamd::bmmw::bmm_wide_kernel<false, false, 3, 3, 0, 2, 7, false, true>"])}
+                                     ["pcamd::bmmw::bmm_wide_kernel<false, false, 3, 3, 0, 2, 7, false, true, false>"])}
 
 
 def pmc_field(workload, kernels, keys):
@@ -802,9 +801,11 @@ def pmc_probe_bmm(torch, dev):
     """Eager launches for rocprofv3 --pmc passes over the BMM kernels, each
     dispatch carrying its own counters: three 256 MiB bf16 copies
     (calibration), then three launches each of config 4 and of the config-5
-    forward, dgrad, wgrad (a_m_b_n) and the layer's K-major wgrad, in that
-    order."""
-    from practice_cuda_amd.impls.hip_per_block import hip_per_block_bmm
+    forward, dgrad, wgrad (a_m_b_n) and the layer's K-major wgrad, then of two
+    K-split products (16 x 14336 x 4096 with K-major B, and 3 x 1001 x 777 x
+    1031, whose rows are not 16-byte aligned; block scales, operands rotating
+    beyond the caches), in that order."""
+    from practice_cuda_amd.impls.hip_per_block import hip_per_block_bmm, hip_per_block_quant
     from practice_cuda_amd.registry import QuantResult
     src = torch.ones(1 << 27, dtype=torch.bfloat16, device=dev)  # 256 MiB
     dst = torch.empty_like(src)
@@ -825,13 +826,27 @@ def pmc_probe_bmm(torch, dev):
     qx_m = q["x_m"]
     qx_mk = QuantResult(qx_m.tensor.transpose(-1, -2).contiguous().transpose(-1, -2), qx_m.dequant_scale,
                         qx_m.impl, "block", dict(qx_m.meta))
-    gemms["wgrad_layer_a_k_b_k"] = lambda i: hip_per_block_bmm(dyt_k, qx_mk, out=outs[2])
+    gemms["wgrad_layer_a_k_b_k"] = lambda i: hip_per_block_bmm(dyt_k, qx_mk, out=outs[2][0])
     for name, fn in gemms.items():
         for i in range(3):
             fn(i)
         torch.cuda.synchronize()
-    print(json.dumps({"copy_bytes_read": (1 << 28), "copy_bytes_written": (1 << 28),
-                      "order": ["copy x3", "config4 x3"] + [f"{k} x3" for k in gemms]}))
+    split = {}
+    for name, bsz, m, n, k, sets, k_major in (("split_decode", 1, 16, 14336, 4096, 8, True),
+                                              ("split_unaligned", 3, 1001, 777, 1031, 96, False)):
+        qa = [hip_per_block_quant(torch.randn(bsz, m, k, device=dev).bfloat16(), block_m=1, block_n=128)
+              for _ in range(sets)]
+        w = torch.randn(bsz, n, k, device=dev).bfloat16().transpose(-1, -2)
+        w = w if k_major else w.contiguous()
+        qb = [hip_per_block_quant(w, block_m=128, block_n=128) for _ in range(sets)]
+        torch.cuda.synchronize()
+        for i in range(3):
+            hip_per_block_bmm(qa[i], qb[i])
+        torch.cuda.synchronize()
+        split[name] = {"bytes_read": bsz * (m * k + k * n), "bytes_written": 2 * bsz * m * n}
+        del qa, qb
+    print(json.dumps({"copy_bytes_read": (1 << 28), "copy_bytes_written": (1 << 28), "split": split,
+                      "order": ["copy x3", "config4 x3"] + [f"{k} x3" for k in [*gemms, *split]]}))
 
 
 def pmc_probe_fused(torch, dev):

@@ -6,6 +6,7 @@ from __future__ import annotations
 
 import json
 import os
+import re
 import subprocess
 import sys
 
@@ -67,3 +68,15 @@ def test_config_inputs_follow_baseline():
     # per-block magnitudes spread over about two decades (log-uniform multipliers in [0.1, 10])
     blk = x3.float().view(32, 128, 56, 128).abs().amax(dim=(1, 3))
     assert blk.max().item() / blk.min().item() > 30
+
+
+def test_counter_guard_names_the_kernels_that_run():
+    """pmc_field compares whole names: the ones bench.py expects have as many template arguments as the
+    kernel has parameters, and the committed counters were taken on them."""
+    with open(os.path.join(ROOT, "practice_cuda_amd", "csrc", "bmm_wide.h")) as fh:
+        params = re.search(r"template <([^>]*)>\s*__global__[^;{]*\bbmm_wide_kernel\(", fh.read()).group(1)
+    for workload, names in bench.CONFIG5_KERNELS.values():
+        for name in names:
+            assert name.count(",") == params.count(","), name
+        assert bench.pmc_field(workload, names, "mfma_busy") is not None, workload
+    assert bench.pmc_field("fwd", "some other kernel", "mfma_busy") is None
