@@ -164,7 +164,8 @@ int pcamd_quant_channel(const void *x, int x_dtype, int64_t batch, int64_t m,
  * pcamd_quant_channel with a workspace of pcamd_quant_channel_workspace()
  * bytes (device memory, 4-byte aligned, contents ignored and overwritten; it
  * may be NULL, and is not needed where the size is 0). With it the per-column
- * scales of a tall tensor take two launches instead of four. Same bytes.
+ * scales of a tall tensor take two launches (three if it is narrow as well)
+ * instead of four. Same bytes.
  * Available from PCAMD_ABI_VERSION 5.
  */
 int64_t pcamd_quant_channel_workspace(int64_t batch, int64_t m, int64_t n,

@@ -143,7 +143,9 @@ PCAMD_DEV void store8_n(uint8_t* p, uint2 v, int64_t nv) {
 
 // max |x| over a chunk's elements. SKIP: NaN elements do not count, whatever
 // the type, as in the element-wise kernels (chunk_amax orders bf16 by its bits,
-// so a NaN there is the largest value).
+// so a NaN there is the largest value). In floats: bf16 [100000, 129] in 128 x
+// 128 blocks 15.8 -> 18.8 us, other shapes level; as signed 16-bit maxima of
+// shifted bits 16.7 there but 3-6 % slower elsewhere.
 template <int DT, bool SKIP>
 PCAMD_DEV float chunk_amax_n(const Chunk<DT>& c) {
   if constexpr (!SKIP) {
@@ -952,11 +954,11 @@ __global__ __launch_bounds__(kThreads) void colchan_zero_kernel(ColArgs a) {
 // reads ([18432, 7168] bf16: 117 -> 106 us for the pair).
 //
 // PARTS (a caller's workspace): a workgroup takes part_rows rows (a multiple of
-// 128, at most 32 such parts per column) and stores its column maxima in its
-// part's row of the workspace; the apply kernel takes the maximum of a
-// column's parts and its first slab writes the scales. Nothing is cleared
-// first and nothing finished afterwards: two launches instead of four. MI355X,
-// bf16 [4096, 14336]: 48.9 -> 45.2 us per call.
+// 128, col_parts) and stores its column maxima in its part's row of the
+// workspace; the apply kernel takes the maximum of a column's parts (of many,
+// after colchan_reduce_kernel) and its first slab writes the scales. Nothing is
+// cleared first and nothing finished afterwards: two or three launches instead
+// of four. MI355X, bf16 [4096, 14336]: 48.9 -> 44.6 us per call.
 template <int DT, bool UA, bool PARTS>
 __global__ __launch_bounds__(kThreads) void colchan_amax_kernel(ColArgs a) {
   constexpr int EB = elem_bytes<DT>();
