@@ -197,7 +197,8 @@ class _Direct:
 
 _PLAIN = (torch.Tensor, nn.Parameter)
 _OPS = (block_scaled_bmm, tensor_scaled_bmm, quant_block, quant_block_dual, quant_tensor)
-_OWN_KERNELS = tuple(op._backend_fns[None] for op in _OPS)
+_KERNELS = tuple(op._backend_fns for op in _OPS)
+_OWN_KERNELS = [fns[None] for fns in _KERNELS]
 # torch.library's record of what was registered on ops from Python
 _REGISTERED = torch.library._impls
 _OVERRIDES = frozenset(f"{op._qualname.replace('::', '/')}/{key}" for op in _OPS
@@ -209,7 +210,7 @@ _dispatch_modes, _function_modes = torch._C._len_torch_dispatch_stack, torch._C.
 _transforms, _recording = torch._C._functorch.peek_interpreter_stack, torch.is_grad_enabled
 
 
-def _ops(*tensors):
+def _ops(*tensors, saved=()):
     """What the layer calls: ``torch.ops.pcamd`` wherever something looks at or
     stands in for the ops (compilation or tracing, a function or dispatch mode
     such as a counter or selective checkpointing, a function transform, a
@@ -217,16 +218,20 @@ def _ops(*tensors):
     the functions they run, which spares eager steps the dispatcher's Python
     layers (6.5 us of host time per op, six ops per step). Either way the same
     launches on the same stream; only called where autograd does not record
-    (inside the autograd function)."""
+    (inside the autograd function). tensors: the call's inputs; saved: results
+    of the ops themselves, which only a saved-tensor hook may have wrapped."""
     if (torch.compiler.is_compiling() or _tracing() is not None or _dispatch_modes() or _function_modes()
             or _recording() or _transforms() is not None or _profiling()
             or not _OVERRIDES.isdisjoint(_REGISTERED)
-            or tuple([op._backend_fns[None] for op in _OPS]) != _OWN_KERNELS):
+            or [fns[None] for fns in _KERNELS] != _OWN_KERNELS):
         return torch.ops.pcamd
     for t in tensors:
         # the dispatcher hands the ops' functions another tensor: it calls the fake implementations for
         # meta tensors and materializes lazy negations and zeros first
         if t is not None and (type(t) not in _PLAIN or t.is_meta or t.is_neg() or t._is_zerotensor()):
+            return torch.ops.pcamd
+    for t in saved:
+        if type(t) not in _PLAIN and t is not None:
             return torch.ops.pcamd
     return _Direct
 
@@ -304,7 +309,7 @@ class _Float8BlockBMMLinearFunction(torch.autograd.Function):
         f8 = config.grad_fp8_dtype or config.fp8_dtype  # dY's format
         dy = grad_output.contiguous()
         saved = ctx.saved_tensors  # once: each access runs the saved-tensor hooks
-        ops = _ops(dy, *saved)
+        ops = _ops(dy, saved=saved)
         grad_input = grad_weight = grad_bias = None
         if config.granularity == "tensor":
             qx, sx, qw, sw = saved

@@ -175,3 +175,16 @@ def test_layer_ops_go_through_the_dispatcher_where_a_kernel_was_registered():
         run = subprocess.run([sys.executable, "-c", prologue + check.format(register)], cwd=root, capture_output=True,
                              text=True, timeout=300)
         assert run.returncode == 0, register + "\n" + run.stderr
+
+
+def test_layer_ops_go_through_the_dispatcher_for_saved_subclasses():
+    """A saved-tensor hook may hand backward something else than what the ops returned."""
+    from practice_cuda_amd.modules import _Direct, _ops
+
+    class Sub(torch.Tensor):
+        pass
+
+    x = torch.zeros(1, 2, 3)
+    with torch.no_grad():
+        assert _ops(x, saved=(x, None, x)) is _Direct
+        assert _ops(x, saved=(x, None, x.as_subclass(Sub))) is torch.ops.pcamd
